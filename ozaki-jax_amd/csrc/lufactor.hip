@@ -13,7 +13,7 @@
 //     diagonal block for its rows c .. c+31 (the U12 block);
 //  3. lu_update_kernel: trailing A22 -= L21 U12, 64 x 64 tiles, K = 32.
 // The panel step is the critical path: 32 pivot searches, one workgroup
-// barrier each.
+// barrier each (about 0.7 us).
 #include <cfloat>
 
 #include "common.h"
@@ -27,7 +27,7 @@ constexpr int kLuPanel = 2 * kLuSub;             // panel width
 constexpr int kLuMaxRows = kLuThreads * kLuRpt;  // panel height the registers hold
 constexpr int kLuPairs = 2 * kLuPanel;           // rows a panel's swaps can move
 constexpr int kLuWaves = kLuThreads / 64;
-constexpr int kLuMapInts = 1 + 2 * kLuPairs;
+constexpr int kLuMapInts = 4 + 2 * kLuPairs;  // (the L block behind them 16-byte aligned)
 
 // ---------------------------------------------------------------- waves
 template <int CTRL>
@@ -57,352 +57,482 @@ __device__ __forceinline__ uint32_t lu_wave_reduce(uint32_t u) {
 
 // ---------------------------------------------------------------- panel
 // The panel's rows stay where they were read: thread t holds physical rows
-// t + i * kLuThreads (relative to row c).  A pivot is not moved in
-// registers; the kernel tracks positions instead (LAPACK's row order after
-// its swaps) and stores every row at its final position.
+// t + i * kLuThreads (relative to row c), i < S.  A pivot is not moved in
+// registers; the kernel keeps what became of each row and stores it at its
+// final position.
+//
+// What bounds it: one workgroup on one CU, 32 dependent column steps.  Each
+// step is a chain of a pivot search, an LDS exchange with one barrier and
+// the rank-1 update.  The steps run as a rolled loop: unrolled over the 32
+// columns the kernel was 28000 instructions, and fetching that much
+// straight-line code (200 KB, over the 64 KB instruction cache) cost about
+// a sixth of every short step and more of the tall ones.  The loop needs the active column
+// in a fixed register, so each step rotates a row's registers by one: the
+// updated columns move down and the finished L entry enters at the end.
+// Measured with the row slots a compile-time count, the loads and stores
+// four lanes a row and the permutation composed in parallel (us a panel,
+// unrolled -> rolled): 4096 rows 108 -> 88, 2048 71 -> 45, 512 46 -> 30; n =
+// 4096 factored in 9.1 ms (12.7).  Four waves (one a SIMD) instead of eight
+// were slower (55 at 2048 rows), reading the pivot row back from LDS instead
+// of by readlane too (50).
 struct LuPanelShared {
-  // per-wave candidates: (|value| bits + 1) << 32 | (INT_MAX - physical row),
-  // so that the largest key is the largest value, then the lowest row
-  uint64_t ckey[2][kLuWaves];
-  float crow[2][kLuWaves][kLuSub];    //   and those rows' sub-panel values
-  float la[kLuSub][kLuSub];           // the first sub-panel's pivot rows
-  float lb[kLuSub][kLuSub];           //   and their second sub-panel columns
-  float u01[kLuSub][kLuSub];          // U block right of the first sub-panel
-  int piv[kLuPanel];                  // position swapped with column j's diagonal
-  int prow_of[kLuPanel];              // physical pivot row of column j
-  int smap[kLuMaxRows];               // position q holds physical row smap[q]
-  int inv[kLuMaxRows];                // physical row x sits at position inv[x]
+  // per-wave candidates: the bits of |value| (0: none) and the physical row
+  uint2 ckey[2][kLuWaves];
+  float crow[2][kLuWaves][kLuSub];      //   and those rows' sub-panel registers
+  float prow[kLuPanel][kLuSub];         // pivot rows: their own sub-panel's columns
+  float b0[kLuSub][kLuSub];             // first sub-panel's pivots: the second's columns
+  float l10[kLuSub][kLuSub];            // second sub-panel's pivots: the first's columns
+  float u01[kLuSub][kLuSub];            // U block right of the first sub-panel
+  int prow_of[kLuPanel];                // physical pivot row of column j
+  int top[kLuPanel];                    // position of displaced row x < w
+  int displaced[kLuPanel];
+  uint32_t pivot_top;                   // bit x: row x < w is a pivot
+  int pos[kLuWaves][64];
+  float4 stage[kLuWaves][64 * kLuSub / 4];
 };
 
-// Partial pivoting on one sub-panel in registers: r[i][k] is column OFF + k
-// of physical row t + i * kLuThreads (rows < m); bit i of `used` marks the
-// rows that are pivots already, and 6-bit field i of pcode receives 1 + the
-// column (OFF + j) a row becomes the pivot of.  Column j's pivot is the unused row with the
-// largest |value| (on ties the lowest row of the lowest lane); it takes
-// position OFF + j, swapping with the row there as LAPACK's getf2 swaps
-// (lu_compose_positions works those out from prow_of).  A zero pivot leaves the
-// column as it is (its unused entries are zero too) and raises
-// OZK_FLAG_SINGULAR.
-template <int OFF>
-__device__ __forceinline__ void lu_factor_sub(float (&r)[kLuRpt][kLuSub], uint32_t& used,
-                                              uint64_t& pcode, int ncols, int m,
-                                              LuPanelShared& sh, uint32_t* status) {
-  const int t = threadIdx.x, wave = t / 64, lane = t % 64;
-  uint32_t present = 0u;  // row slots below the panel's last row
-#pragma unroll
-  for (int i = 0; i < kLuRpt; ++i) present |= (t + i * kLuThreads < m) ? 1u << i : 0u;
-  // (a compile-time column index: the loop body is too large for the
-  // unroller, and a run-time j would index r through scratch memory)
-  static_for<0, kLuSub>([&](auto jc) {
-    constexpr int j = decltype(jc)::value;
-    if (j >= ncols) return;  // uniform
-    const int dj = OFF + j;
-    const int par = j & 1;
-    const uint32_t avail = present & ~used;  // row slots that can still pivot
-    // + 1: an unused row holding 0 still beats a lane with no row (bb = 0)
-    uint32_t bb = 0u;
-    int br = INT_MAX;
-#pragma unroll
-    for (int i = 0; i < kLuRpt; ++i) {
-      if (i * kLuThreads >= m) break;  // uniform: no thread has row slot i
-      const uint32_t bits = __float_as_uint(fabsf(r[i][j])) + 1u;
-      if (((avail >> i) & 1u) && bits > bb) {
-        bb = bits;
-        br = t + i * kLuThreads;
-      }
-    }
-    const uint32_t wb = lu_wave_reduce<true>(bb);
-    const uint64_t tie = __ballot(bb == wb);
-    const int wr = __builtin_amdgcn_readlane(br, (int)__builtin_ctzll(tie));
-    if (lane == 0) sh.ckey[par][wave] = (uint64_t)wb << 32 | (uint32_t)(INT_MAX - wr);
-    if (wr != INT_MAX && lane == (wr & 63)) {  // the candidate's lane
-      const int iw = wr / kLuThreads;          // wave-uniform
-      static_for<0, kLuRpt>([&](auto ic) {
-        constexpr int i = decltype(ic)::value;
-        if (i == iw) {
-          float4* const d = (float4*)sh.crow[par][wave];
-#pragma unroll
-          for (int q = 0; q < kLuSub / 4; ++q)
-            d[q] = make_float4(r[i][4 * q], r[i][4 * q + 1], r[i][4 * q + 2], r[i][4 * q + 3]);
-          // (distinct per case: keeps the compiler from merging the cases
-          // into one store of a run-time-indexed row)
-          asm volatile("; lu candidate row %0" ::"n"(i));
-        }
-      });
-    }
-    __syncthreads();
+// Column `col` of a sub-panel after lu_factor_sub sits in register
+// lu_reg(col): its two rotations (16 wide, then 8 wide) leave the halves
+// swapped.
+constexpr int lu_reg(int col) { return (col + kLuSub / 2) % kLuSub; }
 
-    // all keys first, then the maximum: one LDS round trip
-    uint64_t keys[kLuWaves];
-#pragma unroll
-    for (int q = 0; q < kLuWaves; ++q) keys[q] = sh.ckey[par][q];
-    uint64_t best = keys[0];
-#pragma unroll
-    for (int q = 1; q < kLuWaves; ++q) best = keys[q] > best ? keys[q] : best;
-    const int pr = __builtin_amdgcn_readfirstlane(INT_MAX - (int)(uint32_t)best);
-    const int pw = (pr % kLuThreads) / 64;  // the wave holding that row
-    float prow[kLuSub];
-#pragma unroll
-    for (int k = 0; k < kLuSub; ++k) prow[k] = sh.crow[par][pw][k];
-    if (t == pr % kLuThreads) {  // the pivot's owner; its slot ip is uniform
-      const int ip = pr / kLuThreads;
-      used |= 1u << ip;
-      pcode |= (uint64_t)(dj + 1) << (6 * ip);
-    }
-    if (t == 0) sh.prow_of[dj] = pr;  // positions are composed after the sub-panel
-    const float pv = prow[j];
-    if (pv != 0.0f) {  // uniform
-      // LAPACK's getf2 scales by the reciprocal when it is representable.
-      // Pivot rows (old and new) get l = 0, which leaves them as they are.
-      const bool recip = fabsf(pv) >= FLT_MIN;  // uniform
-      const float rinv = 1.0f / pv;
-      const uint32_t act_bits = avail & ~used;  // the new pivot is out too
-#pragma unroll
-      for (int i = 0; i < kLuRpt; ++i) {
-        if (i * kLuThreads >= m) break;  // uniform
-        const bool act = (act_bits >> i) & 1u;
-        float q;
-        if (recip)  // uniform: the division is only paid for tiny pivots
-          q = r[i][j] * rinv;
-        else
-          q = r[i][j] / pv;
-        const float l = act ? q : 0.0f;
-        r[i][j] = act ? q : r[i][j];
-#pragma unroll
-        for (int k = j + 1; k < kLuSub; ++k) r[i][k] = fmaf(-l, prow[k], r[i][k]);
-      }
-    } else if (t == 0) {
-      atomicOr(status, OZK_FLAG_SINGULAR);
-    }
-  });
+// One dword per lane from global memory into LDS at lds_addr + 4 lane, for
+// the active lanes (as dma16; the reader waits with wait_vm).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lu_dma4(uint32_t lds_addr, const void* gbase, uint32_t voff) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %1, %2"
+      :
+      : "s"(lds_addr), "v"(voff), "s"(gbase)
+      : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+__device__ __forceinline__ float lu_readlane(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// LAPACK's swap sequence of the panel (column j swaps position j with the
-// position its pivot row sits at) composed by wave 0 after the last column:
-// only the physical rows 0 .. 31 and the pivot rows ever move, so lane k
-// follows one of them (lanes 0-31: rows 0-31, lanes 32-63: the pivot row of
-// column k - 32) through the w swaps.  Writes inv[row] and smap[position]
-// for those rows and piv[j], the position column j swapped with.
-__device__ __forceinline__ void lu_compose_positions(int w, int m, LuPanelShared& sh) {
-  const int t = threadIdx.x;
-  if (t >= 64) return;
-  const int pf = t < kLuPanel && t < w ? sh.prow_of[t] : -1;  // lane j: column j's pivot
-  int row = -1;
-  if (t < kLuPanel) {
-    if (t < m) row = t;
-  } else if (t - kLuPanel < w) {
-    row = sh.prow_of[t - kLuPanel];
-  }
-  int pos = row;
-  for (int j = 0; j < w; ++j) {  // uniform
-    const int pr = __builtin_amdgcn_readlane(pf, j);
-    const uint64_t hit = __ballot(row == pr);  // lane kLuPanel + j at least
-    const int pp = __builtin_amdgcn_readlane(pos, (int)__builtin_ctzll(hit));
-    pos = pos == j ? pp : (pos == pp ? j : pos);
-    if (t == 0) sh.piv[j] = pp;
-  }
-  if (row >= 0) {  // a row followed by two lanes gets the same values twice
-    sh.inv[row] = pos;
-    sh.smap[pos] = row;
+// `steps` columns (panel columns dj0 ..) of a sub-panel over the rotating
+// registers 0 .. WD - 1: register 0 holds the active column, registers
+// WD - s .. WD - 1 the L entries of the s columns finished here.  lm[i]: all
+// ones while row slot i can still become a pivot, 0 for a pivot or no row;
+// field i of pcode receives 1 + the panel column a row becomes the pivot of.
+// The pivot is the candidate with the largest |value| (bit patterns: a NaN
+// wins); on ties the lowest wave, slot, lane.  Where every candidate is zero
+// the lowest row is taken, the column left as it is and OZK_FLAG_SINGULAR
+// raised.  fetch(pr, dj) starts the copy of pivot row pr's other sub-panel
+// into LDS (one wave).
+template <int S, int WD, class Fetch>
+__device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)[S],
+                                           uint64_t& pcode, int dj0, int steps,
+                                           LuPanelShared& sh, uint32_t* status, Fetch fetch) {
+  const int t = threadIdx.x, lane = t % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(t / 64);
+  const int k0 = 2 * (lane % kLuWaves);  // the lane's registers of record lane / kLuWaves
+#pragma unroll 1
+  for (int s = 0; s < steps; ++s) {
+    const int dj = dj0 + s, par = dj & 1;
+    uint32_t u[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) u[i] = __float_as_uint(r[i][0]) & lm[i] & 0x7fffffffu;
+    bool zero = false;  // every candidate is 0: choose by row
+    uint2 kv;
+    float2 rv;
+    float pvl;
+    uint32_t best;
+#pragma unroll 1
+    for (;;) {
+      uint32_t mx = u[0];
+#pragma unroll
+      for (int i = 1; i < S; ++i) mx = max(mx, u[i]);
+      // the lane's slot (lowest of equals), while the wave's maximum forms
+      int sel = S - 1;
+#pragma unroll
+      for (int i = S - 2; i >= 0; --i) sel = u[i] == mx ? i : sel;
+      const uint32_t wb = lu_wave_reduce<true>(mx);
+      const int hl = (int)__builtin_ctzll(__ballot(mx == wb));
+      const int slot = S > 1 ? __builtin_amdgcn_readlane(sel, hl) : 0;
+      if (lane == hl) {
+        sh.ckey[par][wave] = make_uint2(wb, (uint32_t)(slot * kLuThreads + t));
+        static_for<0, S>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          if (i == slot) {
+            float4* const d = (float4*)sh.crow[par][wave];
+#pragma unroll
+            for (int q = 0; q < kLuSub / 4; ++q)
+              d[q] = make_float4(r[i][4 * q], r[i][4 * q + 1], r[i][4 * q + 2], r[i][4 * q + 3]);
+            // (distinct per case: keeps the compiler from merging the cases
+            // into one store of a run-time-indexed row)
+            asm volatile("; lu candidate row %0" ::"n"(i));
+          }
+        });
+      }
+      __syncthreads();
+      // Lane l reads key l % 8 and two values of candidate row l / 8, so the
+      // winner's row is there without a second LDS round trip.
+      kv = sh.ckey[par][lane % kLuWaves];
+      pvl = sh.crow[par][lane % kLuWaves][0];
+      rv = *(const float2*)&sh.crow[par][lane / kLuWaves][k0];
+      best = kv.x;
+      best = max(best, lu_dpp<0xB1>(best));   // quad_perm [1, 0, 3, 2]
+      best = max(best, lu_dpp<0x4E>(best));   // quad_perm [2, 3, 0, 1]
+      best = max(best, lu_dpp<0x141>(best));  // half-row mirror: 8 lanes
+      best = __builtin_amdgcn_readfirstlane(best);
+      if (best != 0u || zero) break;  // uniform over the workgroup
+      zero = true;
+#pragma unroll
+      for (int i = 0; i < S; ++i) u[i] = (uint32_t)(INT_MAX - t - kLuThreads * i) & lm[i];
+      __syncthreads();
+    }
+    // LAPACK's getf2 scales by the pivot's reciprocal; below FLT_MIN, where
+    // that can overflow, pivot and column are scaled by 2^24 first (exact).
+    // Every lane inverts its candidate while the maximum forms (the empty
+    // asm keeps the compiler from doing it after the choice instead).
+    float rl = 1.0f / (fabsf(pvl) < FLT_MIN ? pvl * 0x1p24f : pvl);
+    asm volatile("" : "+v"(rl));
+    const int qw = (int)__builtin_ctzll(__ballot(kv.x == best));
+    const int pr = __builtin_amdgcn_readlane((int)kv.y, qw);
+    const float pv = lu_readlane(pvl, qw);
+    float rinv = lu_readlane(rl, qw);
+    if (fabsf(pv) < FLT_MIN) {  // uniform
+      if (pv == 0.0f) {
+        rinv = 0.0f;
+        if (t == 0) atomicOr(status, OZK_FLAG_SINGULAR);
+      } else {
+#pragma unroll
+        for (int i = 0; i < S; ++i) r[i][0] = lm[i] ? r[i][0] * 0x1p24f : r[i][0];
+      }
+    }
+    // the pivot row's columns right of the active one (0 for finished ones)
+    const float px = k0 < WD - s ? rv.x : 0.0f, py = k0 + 1 < WD - s ? rv.y : 0.0f;
+    float p[WD];
+#pragma unroll
+    for (int k = 1; k < WD; ++k) p[k] = lu_readlane(k & 1 ? py : px, qw * kLuWaves + k / 2);
+    if (wave == dj % kLuWaves && lane / kLuWaves == qw) {
+      // the lane's registers of the pivot row, at their columns
+      constexpr int H = kLuSub / 2;
+      const int c0 = WD == kLuSub ? (k0 + s) % kLuSub : (k0 < H ? H + (k0 + s) % H : k0 - H);
+      const int c1 = WD == kLuSub ? (k0 + 1 + s) % kLuSub
+                                  : (k0 < H ? H + (k0 + 1 + s) % H : k0 + 1 - H);
+      sh.prow[dj][c0] = rv.x;
+      sh.prow[dj][c1] = rv.y;
+      if (k0 == 0) sh.prow_of[dj] = pr;
+    }
+    fetch(pr, dj);
+    if (wave == (int)((uint32_t)pr / 64u % kLuWaves)) {  // uniform: the wave of the pivot's owner
+      if (lane == (int)((uint32_t)pr % 64u))
+        pcode |= (uint64_t)(dj + 1) << (6 * ((uint32_t)pr / kLuThreads));
+#pragma unroll
+      for (int i = 0; i < S; ++i) lm[i] = t + i * kLuThreads == pr ? 0u : lm[i];
+    }
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      const uint32_t q = __float_as_uint(r[i][0] * rinv);
+      const float l = __uint_as_float(q & lm[i]);
+      const float keep = __uint_as_float((q & lm[i]) | (__float_as_uint(r[i][0]) & ~lm[i]));
+#pragma unroll
+      for (int k = 1; k < WD; ++k) r[i][k - 1] = fmaf(-l, p[k], r[i][k]);
+      r[i][WD - 1] = keep;
+    }
   }
 }
 
-// Rows i in [I0, I1) of a sub-panel from global: r[i][k] = P[ph * lda +
-// col0 + k] for physical row ph and k < ncols, zero elsewhere.  VEC: 16-byte
-// loads (lda % 4 == 0, 16-byte aligned A; col0 is a multiple of 16).
-template <bool VEC, int I0, int I1>
-__device__ __forceinline__ void lu_load_rows(float (&r)[kLuRpt][kLuSub], const float* P,
-                                             int64_t lda, int col0, int ncols, int m) {
-  const int t = threadIdx.x;
+// Rotates registers 0 .. WD - 1 by `steps` columns that a narrow sub-panel
+// does not have.
+template <int S, int WD>
+__device__ __forceinline__ void lu_rotate(float (&r)[S][kLuSub], int steps) {
+#pragma unroll 1
+  for (int s = 0; s < steps; ++s) {
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      const float f = r[i][0];
+#pragma unroll
+      for (int k = 1; k < WD; ++k) r[i][k - 1] = r[i][k];
+      r[i][WD - 1] = f;
+    }
+  }
+}
+
+// Partial pivoting on one sub-panel of ncols columns (panel columns off ..)
+// in registers: r[i][k] comes in as column k and leaves as column c in
+// register lu_reg(c).  The first 8 columns rotate all 16 registers, the last
+// 8 only the upper columns' (11 FMAs a row and column instead of 15).
+template <int S, class Fetch>
+__device__ __forceinline__ void lu_factor_sub(float (&r)[S][kLuSub], uint32_t (&lm)[S],
+                                              uint64_t& pcode, int off, int ncols,
+                                              LuPanelShared& sh, uint32_t* status,
+                                              Fetch fetch) {
+  constexpr int H = kLuSub / 2;
+  const int n0 = ncols < H ? ncols : H, n1 = ncols - n0;
+  lu_columns<S, kLuSub>(r, lm, pcode, off, n0, sh, status, fetch);
+  if (n0 < H) lu_rotate<S, kLuSub>(r, H - n0);
+  lu_columns<S, H>(r, lm, pcode, off + H, n1, sh, status, fetch);
+  if (n1 < H) lu_rotate<S, H>(r, H - n1);
+}
+
+// Row slots [I0, I1) of a sub-panel from global memory: r[i][k] = P[ph * lda
+// + col0 + k].  VEC (16-byte aligned rows, full panels) reads 16 rows of 64 bytes per
+// load, four lanes a row (one row per lane would touch 64 cache lines a
+// load); lu_load_finish then turns the rows into one per lane through the
+// wave's LDS.  Rows past m are zero.
+template <bool VEC, int I0, int I1, int S>
+__device__ __forceinline__ void lu_load_issue(float (&r)[S][kLuSub], const float* P, int64_t lda,
+                                              int col0, int ncols, int m) {
+  const int t = threadIdx.x, lane = t % 64;
 #pragma unroll
   for (int i = I0; i < I1; ++i) {
-    const int ph = t + i * kLuThreads;
-    const bool live = ph < m;
-    const float* const row = P + (int64_t)(live ? ph : 0) * lda + col0;
-    if (VEC && ncols == kLuSub) {
+    if constexpr (VEC) {
 #pragma unroll
       for (int q = 0; q < kLuSub / 4; ++q) {
-        const float4 v = live ? ((const float4*)row)[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const int ph = i * kLuThreads + (t - lane) + 16 * q + lane / 4;
+        const float4 v = *(const float4*)(P + (int64_t)(ph < m ? ph : 0) * lda + col0 +
+                                          4 * (lane % 4));
         r[i][4 * q] = v.x;
         r[i][4 * q + 1] = v.y;
         r[i][4 * q + 2] = v.z;
         r[i][4 * q + 3] = v.w;
       }
     } else {
+      const int ph = t + i * kLuThreads;
+      const float* const row = P + (int64_t)(ph < m ? ph : 0) * lda + col0;
 #pragma unroll
-      for (int k = 0; k < kLuSub; ++k) r[i][k] = (live && k < ncols) ? row[k] : 0.0f;
+      for (int k = 0; k < kLuSub; ++k) r[i][k] = (ph < m && k < ncols) ? row[k] : 0.0f;
     }
   }
 }
 
-// Stores the rows whose bit in `skip` is clear at position pos(ph).
-template <bool VEC, class Pos>
-__device__ __forceinline__ void lu_store_rows(const float (&r)[kLuRpt][kLuSub], float* P,
-                                              int64_t lda, int col0, int ncols, int m,
-                                              uint32_t skip, Pos pos) {
-  const int t = threadIdx.x;
+// 16-byte unit of (row, quarter of its 64 bytes) in a wave's stage: the
+// quarters rotate with row / 4, which spreads both access patterns over the
+// banks.
+__device__ __forceinline__ int lu_stage(int row, int q) { return 4 * row + (q ^ ((row / 4) % 4)); }
+
+template <bool VEC, int I0, int I1, int S>
+__device__ __forceinline__ void lu_load_finish(float (&r)[S][kLuSub], int ncols, int m,
+                                               LuPanelShared& sh) {
+  if (!VEC) return;
+  const int t = threadIdx.x, lane = t % 64;
+  float4* const st = sh.stage[t / 64];
 #pragma unroll
-  for (int i = 0; i < kLuRpt; ++i) {
-    const int ph = t + i * kLuThreads;
-    if (ph >= m || ((skip >> i) & 1u)) continue;
-    float* const row = P + (int64_t)pos(ph) * lda + col0;
-    if (VEC && ncols == kLuSub) {
+  for (int i = I0; i < I1; ++i) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-      for (int q = 0; q < kLuSub / 4; ++q)
-        ((float4*)row)[q] = make_float4(r[i][4 * q], r[i][4 * q + 1], r[i][4 * q + 2],
-                                        r[i][4 * q + 3]);
-    } else {
+    for (int q = 0; q < 4; ++q)
+      st[lu_stage(16 * q + lane / 4, lane % 4)] =
+          make_float4(r[i][4 * q], r[i][4 * q + 1], r[i][4 * q + 2], r[i][4 * q + 3]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const bool live = t + i * kLuThreads < m;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4 v = st[lu_stage(lane, q)];
+      r[i][4 * q] = live ? v.x : 0.0f;
+      r[i][4 * q + 1] = live ? v.y : 0.0f;
+      r[i][4 * q + 2] = live ? v.z : 0.0f;
+      r[i][4 * q + 3] = live ? v.w : 0.0f;
+    }
+  }
+}
+
+// Stores a factored sub-panel's rows, row slot i of this lane at position
+// pos(i) (negative: not stored), through the wave's LDS as the loads.
+template <bool VEC, int S, class Pos>
+__device__ __forceinline__ void lu_store_rows(const float (&r)[S][kLuSub], float* P, int64_t lda,
+                                              int col0, int ncols, LuPanelShared& sh, Pos pos) {
+  const int t = threadIdx.x, lane = t % 64;
+  float4* const st = sh.stage[t / 64];
+  int* const ps = sh.pos[t / 64];
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    const int at = pos(i);
+    if constexpr (VEC) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      ps[lane] = at;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = lu_reg(4 * q);
+        st[lu_stage(lane, q)] = make_float4(r[i][k], r[i][k + 1], r[i][k + 2], r[i][k + 3]);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = 16 * q + lane / 4, to = ps[row];
+        const float4 v = st[lu_stage(row, lane % 4)];
+        if (to >= 0) *(float4*)(P + (int64_t)to * lda + col0 + 4 * (lane % 4)) = v;
+      }
+    } else if (at >= 0) {
+      float* const row = P + (int64_t)at * lda + col0;
 #pragma unroll
       for (int k = 0; k < kLuSub; ++k)
-        if (k < ncols) row[k] = r[i][k];
+        if (k < ncols) row[k] = r[i][lu_reg(k)];
     }
   }
 }
 
 // b[i] -= a[i] U01 for the rows that are not pivots of the first sub-panel,
 // i in [I0, I1).
-template <int I0, int I1>
-__device__ __forceinline__ void lu_update_rows(float (&b)[kLuRpt][kLuSub],
-                                               const float (&a)[kLuRpt][kLuSub], int m,
-                                               uint32_t used, const LuPanelShared& sh) {
-  const int t = threadIdx.x;
+template <int I0, int I1, int S>
+__device__ __forceinline__ void lu_update_rows(float (&b)[S][kLuSub], const float (&a)[S][kLuSub],
+                                               const uint32_t (&lm)[S], const LuPanelShared& sh) {
 #pragma unroll
-  for (int i = I0; i < I1; ++i) {
-    const int ph = t + i * kLuThreads;
-    if (ph >= m || ((used >> i) & 1u)) continue;
+  for (int q = 0; q < kLuSub; ++q) {
+    asm volatile("" ::: "memory");  // one row of U01 at a time in registers
+    float u[kLuSub];
 #pragma unroll
-    for (int q = 0; q < kLuSub; ++q) {
-      const float l = a[i][q];
+    for (int k = 0; k < kLuSub; ++k) u[k] = sh.u01[q][k];
 #pragma unroll
-      for (int k = 0; k < kLuSub; ++k) b[i][k] = fmaf(-l, sh.u01[q][k], b[i][k]);
+    for (int i = I0; i < I1; ++i) {
+      const float l = __uint_as_float(__float_as_uint(a[i][lu_reg(q)]) & lm[i]);
+#pragma unroll
+      for (int k = 0; k < kLuSub; ++k) b[i][k] = fmaf(-l, u[k], b[i][k]);
     }
   }
 }
 
-// Factors panel columns [c, c + w) over rows [c, n) (m = n - c <= kLuMaxRows
-// rows, w <= kLuPanel) and writes the row permutation its swaps make to
-// maps: maps[0] = w, then kLuPairs destination rows (absolute, -1 = unused)
-// and kLuPairs source rows.  Entries e < w are the diagonal positions c + e;
-// entries kLuPanel + j are the positions column j's swap exchanged with the
-// diagonal, when they lie below the diagonal block.
-template <bool VEC>
+// Factors panel columns [c, c + w) over rows [c, n) (m = n - c <= S *
+// kLuThreads rows, w <= kLuPanel) and writes to maps the row permutation its
+// swaps make: maps[0] = w, then kLuPairs destination rows (absolute, -1 =
+// unused) and kLuPairs source rows.  Entries e < w are the diagonal
+// positions c + e; entry kLuPanel + j puts one of the rows c .. c + w - 1
+// that is no pivot at the place column j's pivot row came from.  Behind them
+// lies the panel's L block (rows c .. c + w - 1, kLuPanel x kLuPanel, zero on
+// and above the diagonal).  The first sub-panel's columns are stored with
+// their rows where they were; the row fix moves them with the columns left of the panel.
+//
+// Up to S = kLuPreload row slots the second sub-panel's loads are issued
+// before the first is factored; above, the registers hold them in two halves
+// after it.
+constexpr int kLuPreload = 4;
+
+template <bool VEC, int S>
 __global__ __launch_bounds__(kLuThreads) void lu_panel_kernel(float* __restrict__ A,
-                                                              int64_t lda, int n, int c, int w,
+                                                              int64_t lda, int n, int c, int cols,
                                                               int* __restrict__ maps,
                                                               uint32_t* __restrict__ status) {
   __shared__ LuPanelShared sh;
-  const int t = threadIdx.x;
+  const int w = VEC ? kLuPanel : cols;
+  const int t = threadIdx.x, lane = t % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(t / 64);
   const int m = n - c;
   const int w0 = w < kLuSub ? w : kLuSub, w1 = w - w0;
   float* const P = A + (int64_t)c * lda + c;
-  for (int q = t; q < m; q += kLuThreads) {  // (ordered by lu_factor_sub's barriers)
-    sh.smap[q] = q;
-    sh.inv[q] = q;
-  }
-  uint32_t used = 0u;
+  if (t == 0) sh.pivot_top = 0u;  // (ordered by the columns' barriers)
   uint64_t pcode = 0u;
+  uint32_t lm[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) lm[i] = t + i * kLuThreads < m ? ~0u : 0u;
 
-  float a[kLuRpt][kLuSub];
-  lu_load_rows<VEC, 0, kLuRpt>(a, P, lda, 0, w0, m);
-  lu_factor_sub<0>(a, used, pcode, w0, m, sh, status);
-  // The first sub-panel's columns go back to the rows they came from; the
-  // panel's permutation moves them at the end.
-  lu_store_rows<VEC>(a, P, lda, 0, w0, m, 0u, [](int ph) { return ph; });
+  float a[S][kLuSub], b[S][kLuSub];
+  lu_load_issue<VEC, 0, S>(a, P, lda, 0, w0, m);
+  if (S <= kLuPreload && w1 > 0) lu_load_issue<VEC, 0, S>(b, P, lda, kLuSub, w1, m);
+  lu_load_finish<VEC, 0, S>(a, w0, m, sh);
+  // wave 7 copies each pivot row's second sub-panel columns (still as they
+  // came) into b0 for the U01 block
+  const uint32_t lds_b0 = lds_offset(sh.b0), lds_l10 = lds_offset(sh.l10);
+  lu_factor_sub<S>(a, lm, pcode, 0, w0, sh, status, [&](int pr, int dj) {
+    if (wave == kLuWaves - 1 && lane < w1)
+      lu_dma4(__builtin_amdgcn_readfirstlane(lds_b0 + dj * kLuSub * 4),
+              P + (int64_t)pr * lda + kLuSub, 4u * (uint32_t)lane);
+  });
+  lu_store_rows<VEC>(a, P, lda, 0, w0, sh, [&](int i) {
+    return t + i * kLuThreads < m ? t + i * kLuThreads : -1;
+  });
 
-  const uint32_t used0 = used;
-  float b[kLuRpt][kLuSub];
   if (w1 > 0) {
+    if (wave == kLuWaves - 1) wait_vm<0>();
+    __syncthreads();  // b0 and the first sub-panel's pivot rows in LDS
+    if (t < kLuSub) {
+      // U01 = L00^-1 B0; lane k holds column k (zeros past w1)
+      float u[kLuSub];
 #pragma unroll
-    for (int i = 0; i < kLuRpt; ++i) {
-      const int col = (int)((pcode >> (6 * i)) & 63u) - 1;
-      if (col >= 0) {  // a pivot row of the first sub-panel: its L part
-#pragma unroll
-        for (int k = 0; k < kLuSub; ++k) sh.la[col][k] = a[i][k];
-      }
-    }
-    __syncthreads();  // pivot rows staged; prow_of of the first sub-panel final
-    if (t < 64) {
-      // U01 = L00^-1 B0; lane j holds column j's pivot row (position j),
-      // whose second sub-panel columns nothing has changed yet
-      const int jl = t < kLuSub ? t : 0;
-      const float* const src = P + (int64_t)sh.prow_of[jl] * lda + kLuSub;
-      float lrow[kLuSub], u[kLuSub];
-#pragma unroll
-      for (int k = 0; k < kLuSub; ++k) {
-        lrow[k] = sh.la[jl][k];
-        u[k] = k < w1 ? src[k] : 0.0f;
-      }
+      for (int q = 0; q < kLuSub; ++q) u[q] = t < w1 ? sh.b0[q][t] : 0.0f;
 #pragma unroll
       for (int q = 0; q < kLuSub; ++q) {
 #pragma unroll
-        for (int k = 0; k < kLuSub; ++k) {
-          const float uq = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(u[k]), q));
-          if (t > q && t < kLuSub) u[k] = fmaf(-lrow[q], uq, u[k]);
-        }
+        for (int k = q + 1; k < kLuSub; ++k) u[k] = fmaf(-sh.prow[k][q], u[q], u[k]);
       }
-      if (t < kLuSub) {
 #pragma unroll
-        for (int k = 0; k < kLuSub; ++k) sh.u01[t][k] = u[k];
+      for (int q = 0; q < kLuSub; ++q) {
+        sh.u01[q][t] = u[q];
       }
     }
     __syncthreads();  // U01 in LDS
-    // Half of the rows at a time, so that a and b do not both fill the
-    // registers.  The first sub-panel's pivot rows are loaded but left alone.
-    lu_load_rows<VEC, 0, kLuRpt / 2>(b, P, lda, kLuSub, w1, m);
-    lu_update_rows<0, kLuRpt / 2>(b, a, m, used0, sh);
-    lu_load_rows<VEC, kLuRpt / 2, kLuRpt>(b, P, lda, kLuSub, w1, m);
-    lu_update_rows<kLuRpt / 2, kLuRpt>(b, a, m, used0, sh);
-    lu_factor_sub<kLuSub>(b, used, pcode, w1, m, sh, status);  // its barriers follow every load
+    if constexpr (S <= kLuPreload) {
+      lu_load_finish<VEC, 0, S>(b, w1, m, sh);
+      lu_update_rows<0, S>(b, a, lm, sh);
+    } else {
+      // Half of the rows at a time, so that a and b do not both fill the
+      // registers.
+      lu_load_issue<VEC, 0, S / 2>(b, P, lda, kLuSub, w1, m);
+      lu_load_finish<VEC, 0, S / 2>(b, w1, m, sh);
+      lu_update_rows<0, S / 2>(b, a, lm, sh);
+      asm volatile("" ::: "memory");  // the first half's registers of a are free now
+      lu_load_issue<VEC, S / 2, S>(b, P, lda, kLuSub, w1, m);
+      lu_load_finish<VEC, S / 2, S>(b, w1, m, sh);
+      lu_update_rows<S / 2, S>(b, a, lm, sh);
+    }
+    // wave 7 copies each pivot row's L entries of the first sub-panel, as
+    // stored above, into l10
+    lu_factor_sub<S>(b, lm, pcode, kLuSub, w1, sh, status, [&](int pr, int dj) {
+      if (wave == kLuWaves - 1 && lane < kLuSub)
+        lu_dma4(__builtin_amdgcn_readfirstlane(lds_l10 + (dj - kLuSub) * kLuSub * 4),
+                P + (int64_t)pr * lda, 4u * (uint32_t)lane);
+    });
     if (t < kLuSub) {  // positions 0 .. 15 hold the first sub-panel's pivots
 #pragma unroll
-      for (int k = 0; k < kLuSub; ++k)
-        if (k < w1) P[(int64_t)t * lda + kLuSub + k] = sh.u01[t][k];
+      for (int q = 0; q < kLuSub; ++q)
+        if (t < w1) P[(int64_t)q * lda + kLuSub + t] = sh.u01[q][t];
     }
+    if (wave == kLuWaves - 1) wait_vm<0>();
   }
-  __syncthreads();  // prow_of final; the first sub-panel's stores done
-  lu_compose_positions(w, m, sh);
-  __syncthreads();  // inv, smap and piv final
-  if (w1 > 0)
-    lu_store_rows<VEC>(b, P, lda, kLuSub, w1, m, used0, [&](int ph) { return sh.inv[ph]; });
-
-  // The first sub-panel's columns of the rows the permutation moves:
-  // position q takes physical row smap[q].  Load all, then store.
-  int dst = -1, src = 0;
-  if (t < kLuPairs) {
+  __syncthreads();  // prow_of, prow and l10 final
+  // The permutation: position j takes pivot row j; the rows below w that are
+  // no pivots, in order, take the places the pivots from w on leave.
+  const bool col = t < w;
+  const int pj = col ? sh.prow_of[t] : -1;
+  if (wave == 0) {
+    if (col && pj < w) atomicOr(&sh.pivot_top, 1u << pj);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const uint32_t piv = sh.pivot_top;
+    if (col) sh.top[t] = t;
+    if (col && !((piv >> t) & 1u))
+      sh.displaced[__popc(~piv & ((1u << t) - 1u))] = t;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const uint64_t vac = __ballot(col && pj >= w);
+    int dst = -1, src = 0;
+    if (col && pj >= w) {
+      dst = pj;
+      src = sh.displaced[__popcll(vac & ((1ull << t) - 1ull))];
+      sh.top[src] = dst;
+    }
     if (t < kLuPanel) {
-      if (t < w) {
-        dst = t;
-        src = sh.smap[t];
-      }
-    } else if (t - kLuPanel < w) {
-      const int p = sh.piv[t - kLuPanel];
-      if (p >= w) {
-        dst = p;
-        src = sh.smap[p];
-      }
+      maps[1 + t] = col ? c + t : -1;
+      maps[1 + kLuPairs + t] = c + (col ? pj : 0);
+      maps[1 + kLuPanel + t] = dst >= 0 ? c + dst : -1;
+      maps[1 + kLuPairs + kLuPanel + t] = c + src;
     }
-    maps[1 + t] = dst >= 0 ? c + dst : -1;
-    maps[1 + kLuPairs + t] = c + src;
+    if (t == 0) maps[0] = w;
   }
-  if (t == 0) maps[0] = w;
-  // thread t moves entry t % kLuPairs, columns (t / kLuPairs) * 2 and + 1
-  static_assert(kLuThreads * 2 == kLuPairs * kLuSub, "one thread per two elements");
-  __shared__ int dst_s[kLuPairs], src_s[kLuPairs];
-  if (t < kLuPairs) {
-    dst_s[t] = dst;
-    src_s[t] = src;
+  float* const L = (float*)(maps + kLuMapInts);
+#pragma unroll
+  for (int e = t; e < kLuPanel * kLuPanel; e += kLuThreads) {
+    const int rr = e / kLuPanel, cc = e % kLuPanel;
+    float v = 0.0f;
+    if (cc < rr && rr < w)
+      v = rr < kLuSub ? sh.prow[rr][cc]
+                      : (cc < kLuSub ? sh.l10[rr - kLuSub][cc] : sh.prow[rr][cc - kLuSub]);
+    L[e] = v;
   }
-  __syncthreads();
-  const int e = t % kLuPairs, k0 = (t / kLuPairs) * 2;
-  const int de = dst_s[e], se = src_s[e];
-  float v[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    v[k] = (de >= 0 && k0 + k < w0) ? P[(int64_t)se * lda + k0 + k] : 0.0f;
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    if (de >= 0 && k0 + k < w0) P[(int64_t)de * lda + k0 + k] = v[k];
+  if (w1 > 0) {
+    __syncthreads();  // top final
+    lu_store_rows<VEC>(b, P, lda, kLuSub, w1, sh, [&](int i) {
+      const int ph = t + i * kLuThreads, code = (int)((pcode >> (6 * i)) & 63u);
+      if (ph >= m || (code > 0 && code <= kLuSub)) return -1;  // U01's rows are stored above
+      if (code > 0) return code - 1;
+      return ph < w ? sh.top[ph < kLuPanel ? ph : 0] : ph;
+    });
+  }
 }
 
 // The columns outside the panel [c, c + w), 64 per workgroup (lane = column,
@@ -422,7 +552,8 @@ __global__ __launch_bounds__(kLuFixThreads) void lu_rowfix_trsm_kernel(
   const int t = threadIdx.x, lane = t % 64, wv = t / 64;
   const int w = maps[0];
   const int right = n - c - w;
-  const int nleft = (c + kLuFixCols - 1) / kLuFixCols;
+  const int left = c + (w < kLuSub ? w : kLuSub);  // and the first sub-panel's columns
+  const int nleft = (left + kLuFixCols - 1) / kLuFixCols;
   const int nright = (right + kLuFixCols - 1) / kLuFixCols;
   constexpr int kPer = kLuPairs / (kLuFixThreads / 64);  // entries per wave
 
@@ -437,12 +568,11 @@ __global__ __launch_bounds__(kLuFixThreads) void lu_rowfix_trsm_kernel(
   const bool is_right = (int)blockIdx.x >= nleft;
   const int64_t x = is_right ? (int64_t)c + w + ((int)blockIdx.x - nleft) * kLuFixCols + lane
                              : (int64_t)blockIdx.x * kLuFixCols + lane;
-  const bool live = is_right ? x < n : x < c;
+  const bool live = is_right ? x < n : x < left;
   if (is_right) {
-    for (int q = t; q < kLuPanel * kLuPanel; q += kLuFixThreads) {
-      const int rr = q / kLuPanel, cc = q % kLuPanel;
-      L[rr][cc] = (cc < rr && rr < w) ? A[(int64_t)(c + rr) * lda + c + cc] : 0.0f;
-    }
+    const float* const Lg = (const float*)(maps + kLuMapInts);
+    for (int q = t; q < kLuPanel * kLuPanel; q += kLuFixThreads)
+      L[q / kLuPanel][q % kLuPanel] = Lg[q];
   }
   float v[kPer];
   int dst[kPer];
@@ -554,18 +684,38 @@ __global__ void lu_iota_kernel(int32_t* p, int n) {
 }
 
 int64_t lu_factor_max_n() { return kLuMaxRows; }
-size_t lu_factor_workspace_bytes() { return kLuMapInts * sizeof(int); }
+size_t lu_factor_workspace_bytes() {
+  return kLuMapInts * sizeof(int) + kLuPanel * kLuPanel * sizeof(float);
+}
+
+// The panel kernel with as many row slots per thread as the rows need.
+template <bool VEC, int S>
+static void launch_lu_panel(float* A, int64_t lda, int n, int c, int w, int* maps,
+                            uint32_t* status, hipStream_t st) {
+  if constexpr (S > 1) {
+    if (n - c <= (S - 1) * kLuThreads) {
+      launch_lu_panel<VEC, S - 1>(A, lda, n, c, w, maps, status, st);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((lu_panel_kernel<VEC, S>), dim3(1), dim3(kLuThreads), 0, st, A, lda, n, c,
+                     w, maps, status);
+}
 
 template <bool VEC>
 static int lu_factor_steps(float* A, int64_t lda, int n, int32_t* perm, int* maps,
                            uint32_t* status, hipStream_t st) {
   for (int c = 0; c < n; c += kLuPanel) {
     const int w = n - c < kLuPanel ? n - c : kLuPanel;
-    hipLaunchKernelGGL(lu_panel_kernel<VEC>, dim3(1), dim3(kLuThreads), 0, st, A, lda, n, c,
-                       w, maps, status);
+    if (VEC && w == kLuPanel)
+      launch_lu_panel<true, kLuRpt>(A, lda, n, c, w, maps, status, st);
+    else
+      launch_lu_panel<false, kLuRpt>(A, lda, n, c, w, maps, status, st);
     OZK_LAUNCH_CHECK();
     const int right = n - c - w;
-    const int groups = (c + kLuFixCols - 1) / kLuFixCols + (right + kLuFixCols - 1) / kLuFixCols;
+    const int left = c + (w < kLuSub ? w : kLuSub);
+    const int groups =
+        (left + kLuFixCols - 1) / kLuFixCols + (right + kLuFixCols - 1) / kLuFixCols;
     hipLaunchKernelGGL(lu_rowfix_trsm_kernel, dim3(groups + 1), dim3(kLuFixThreads), 0, st, A,
                        lda, n, c, maps, perm);
     OZK_LAUNCH_CHECK();

@@ -254,6 +254,50 @@ def test_lu_factor_pa_equals_lu(ozk, n, pad):
         assert np.array_equal(ps, perm), "pivots differ from sgetrf"
 
 
+def check_lu(A32, F, perm):
+    """P A = L U to the bound of the module's docstring, |L| <= 1."""
+    n = A32.shape[0]
+    assert sorted(perm.tolist()) == list(range(n)), "perm"
+    L = np.tril(F.astype(np.float64), -1) + np.eye(n)
+    U = np.triu(F.astype(np.float64))
+    assert np.abs(np.tril(F, -1)).max(initial=0.0) <= 1.0, "|L| <= 1"
+    err = np.abs(A32.astype(np.float64)[perm] - L @ U).max()
+    assert err <= 8 * n * np.finfo(np.float32).eps * np.abs(A32).max(), err
+
+
+# 512 rows a register slot: first panels of exactly 1, 2 and 5 slots and one
+# row more, last panels of 1, 15, 16, 17 and 31 columns, 16-byte rows or not
+@pytest.mark.parametrize("n,pad", [(15, 1), (31, 0), (49, 3), (512, 0), (513, 3), (1024, 0),
+                                   (1039, 1), (1040, 0), (2560, 0), (2561, 3)])
+def test_lu_factor_row_slot_edges(ozk, n, pad):
+    A32 = np.random.RandomState(300 + n).randn(n, n).astype(np.float32)
+    case(f"ozk_lu_factor_f32 n={n} lda=n+{pad} (slot and panel edges)")
+    F, perm, flags = gpu_factor(A32, pad)
+    assert flags == 0
+    check_lu(A32, F, perm)
+
+
+def test_lu_factor_subnormal_pivots_and_ties(ozk):
+    """Columns whose pivots lie below FLT_MIN (their reciprocals can
+    overflow) and columns of equal magnitudes: still a valid factorisation.
+    The subnormal columns' entries round at 2^-149 each, so their bound is
+    n steps of that."""
+    rng = np.random.RandomState(8)
+    n = 70
+    A32 = np.triu(rng.randn(n, n)).astype(np.float32)
+    A32[:, 5] *= np.float32(1e-40)
+    A32[5, 5], A32[60, 5] = np.float32(1e-42), np.float32(3e-42)
+    A32[20:, 20] = np.where(rng.rand(n - 20) < 0.5, np.float32(1), np.float32(-1))
+    case("ozk_lu_factor_f32 subnormal pivots and ties")
+    F, perm, flags = gpu_factor(A32)
+    assert flags == 0 and np.isfinite(F).all()
+    check_lu(A32, F, perm)
+    L = np.tril(F.astype(np.float64), -1) + np.eye(n)
+    U = np.triu(F.astype(np.float64))
+    err = np.abs(A32.astype(np.float64)[perm] - L @ U)[:, 5].max()
+    assert err <= n * 2.0 ** -149, err
+
+
 def test_lu_factor_singular_flag(ozk):
     from ozaki_jax_amd import _lib
     rng = np.random.RandomState(7)
