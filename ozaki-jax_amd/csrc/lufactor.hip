@@ -197,15 +197,6 @@ __device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)
     const int pr = __builtin_amdgcn_readlane((int)kv.y, qw);
     const float pv = lu_readlane(pvl, qw);
     float rinv = lu_readlane(rl, qw);
-    if (fabsf(pv) < FLT_MIN) {  // uniform
-      if (pv == 0.0f) {
-        rinv = 0.0f;
-        if (t == 0) atomicOr(status, OZK_FLAG_SINGULAR);
-      } else {
-#pragma unroll
-        for (int i = 0; i < S; ++i) r[i][0] = lm[i] ? r[i][0] * 0x1p24f : r[i][0];
-      }
-    }
     // the pivot row's columns right of the active one (0 for finished ones)
     const float px = k0 < WD - s ? rv.x : 0.0f, py = k0 + 1 < WD - s ? rv.y : 0.0f;
     float p[WD];
@@ -227,6 +218,15 @@ __device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)
         pcode |= (uint64_t)(dj + 1) << (6 * ((uint32_t)pr / kLuThreads));
 #pragma unroll
       for (int i = 0; i < S; ++i) lm[i] = t + i * kLuThreads == pr ? 0u : lm[i];
+    }
+    if (fabsf(pv) < FLT_MIN) {  // uniform
+      if (pv == 0.0f) {
+        rinv = 0.0f;
+        if (t == 0) atomicOr(status, OZK_FLAG_SINGULAR);
+      } else {  // (the pivot row itself is out of lm by now)
+#pragma unroll
+        for (int i = 0; i < S; ++i) r[i][0] = lm[i] ? r[i][0] * 0x1p24f : r[i][0];
+      }
     }
 #pragma unroll
     for (int i = 0; i < S; ++i) {
