@@ -57,6 +57,8 @@ extern "C" {
  * OZK_PIPE_ONDEVICE_BF16 to get those values; the 2Sum order turns every
  * non-finite product into NaN, so its results are exact either way. */
 #define OZK_FLAG_INF_SLICE 8u
+/* Set in a published flag word (ozk_matmul_flag_word), never in a device one. */
+#define OZK_FLAGS_READY 0x80000000u
 
 /* Exponent stored for a slice that INT8 planes cannot represent.  The
  * reference's FP32 extraction (extract.py:130-148) gives a line non-finite
@@ -310,6 +312,24 @@ int ozk_matmul_early_flags(const double* A, int64_t lda, const double* B,
                            size_t workspace_bytes, uint32_t* flags,
                            uint32_t* host_flags, void* event, void* stream);
 
+/* ozk_matmul with its flags published by the GEMM itself, for callers that
+ * keep the two words (no counterpart in the reference).  zero_flags: a device
+ * word holding 0, which holds 0 again once the flags are published;
+ * host_word: pinned host memory holding 0, which receives the call's flags |
+ * OZK_FLAGS_READY when the extraction has run and the GEMM starts.  Against
+ * ozk_matmul_early_flags this saves a clearing kernel, a copy and an event.
+ * Both words belong to one call at a time; after an error neither may be used
+ * again.  ozk_wait_flag_word waits for a published word and returns its flags;
+ * it ends with OZK_ERR_HIP on a stream that failed, is being captured or drained
+ * without publishing. */
+int ozk_matmul_flag_word(const double* A, int64_t lda, const double* B,
+                         int64_t ldb, double* C, int64_t ldc, int64_t N,
+                         int64_t K, int64_t M, int pipeline, int n_hi,
+                         int n_lo, int order, void* workspace,
+                         size_t workspace_bytes, uint32_t* zero_flags,
+                         uint32_t* host_word, void* stream);
+int ozk_wait_flag_word(const uint32_t* host_word, void* stream, uint32_t* flags);
+
 /* ozk_matmul without a workspace argument, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  The
@@ -344,6 +364,12 @@ int ozk_gram_early_flags(const double* A, int64_t lda, int64_t rows,
                          int64_t ldg, void* workspace, size_t workspace_bytes,
                          uint32_t* flags, uint32_t* host_flags, void* event,
                          void* stream);
+
+/* ozk_gram with its flags published as ozk_matmul_flag_word's. */
+int ozk_gram_flag_word(const double* A, int64_t lda, int64_t rows,
+                       int64_t cols, int n_hi, int n_lo, double* G,
+                       int64_t ldg, void* workspace, size_t workspace_bytes,
+                       uint32_t* zero_flags, uint32_t* host_word, void* stream);
 
 /* residual(A, x, b, mode="ozaki"): r = b - Ozaki(A, x) in order 2SUM with
  * rho = ozk_rho_f32(K); x is K x ncols, b and r are N x ncols

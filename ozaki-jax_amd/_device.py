@@ -74,6 +74,54 @@ _early_free = {}
 _early_lock = threading.Lock()
 
 
+# Flag word pairs (ozk_matmul_flag_word) per device: a call takes one for the
+# time until its flags have been read, so calls of any threads and streams
+# never share one.  At most _FLAG_WORDS_KEPT of a device's wait for reuse.
+_flag_words_free = {}
+_FLAG_WORDS_KEPT = 64
+
+
+class FlagWords:
+    """A zeroed device word, which collects a call's flags, and the pinned
+    host word that the call's GEMM publishes them to.  run(call, stream) makes
+    the call and returns its flags once they are published; the product may
+    still be queued then.  After an error the pair is not used again, since
+    what was queued may still write it."""
+
+    def __init__(self, device):
+        rt = _hip._rt()
+        self.device = device
+        self.host = rt.host_malloc(4)
+        self.dev = rt.malloc(4)
+        rt.memset(self.dev, 0, 4)
+        rt.sync()
+        self.word = ctypes.c_uint32.from_address(self.host)
+
+    @classmethod
+    def take(cls, device):
+        with _early_lock:
+            free = _flag_words_free.get(device)
+            if free:
+                return free.pop()
+        return cls(device)
+
+    def run(self, call, stream):
+        lib = _lib.load()
+        self.word.value = 0
+        _lib.check(call(self.dev, self.host))
+        fl = ctypes.c_uint32()
+        _lib.check(lib.ozk_wait_flag_word(self.host, stream, ctypes.byref(fl)))
+        with _early_lock:
+            free = _flag_words_free.setdefault(self.device, [])
+            if len(free) < _FLAG_WORDS_KEPT:
+                free.append(self)
+                return fl.value
+        rt = _hip._rt()
+        rt.free(self.dev)
+        rt.host_free(self.host)
+        return fl.value
+
+
 class _TorchFamily:
     """Torch tensors on torch's current device and stream."""
 
@@ -148,6 +196,9 @@ class _TorchFamily:
 
         return word, ev, read
 
+    def flag_words(self):
+        return FlagWords.take(self.dev.index)  # dev is the current device
+
     def read_flags(self, f):
         """Synchronising read of a device flag word."""
         return int(f.item()) & 0xffffffff
@@ -202,6 +253,9 @@ class _HipFamily:
 
     def zeros(self, shape, dtype):
         return _hip.DeviceArray.zeros(shape, dtype)
+
+    def flag_words(self):
+        return FlagWords.take(_hip._rt().device())
 
     def read_flags(self, f):
         return int(f.numpy()[0]) & 0xffffffff

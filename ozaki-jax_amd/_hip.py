@@ -60,6 +60,7 @@ class _Runtime:
                            ("hipStreamSynchronize", [vp]),
                            ("hipStreamCreateWithFlags", [ctypes.POINTER(vp), ctypes.c_uint]),
                            ("hipGetDeviceCount", [ctypes.POINTER(i)]),
+                           ("hipGetDevice", [ctypes.POINTER(i)]),
                            ("hipGetLastError", [])]:
             fn = getattr(h, name)
             fn.restype = i
@@ -81,6 +82,11 @@ class _Runtime:
             self.h.hipGetLastError()  # clear the sticky "no device" status
             return 0
         return n.value
+
+    def device(self):
+        d = ctypes.c_int(0)
+        self.check(self.h.hipGetDevice(ctypes.byref(d)), "hipGetDevice")
+        return d.value
 
     def malloc(self, nbytes):
         p = ctypes.c_void_p()
@@ -105,6 +111,9 @@ class _Runtime:
         p = ctypes.c_void_p()
         self.check(self.h.hipHostMalloc(ctypes.byref(p), nbytes, 0), f"hipHostMalloc({nbytes})")
         return p.value
+
+    def host_free(self, p):
+        self.check(self.h.hipHostFree(p), "hipHostFree")
 
     def copy_async(self, dst, src, nbytes, kind):
         self.check(self.h.hipMemcpyAsync(dst, src, nbytes, kind, None), "hipMemcpyAsync")

@@ -117,6 +117,10 @@ SIGNATURES = {
                                         _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int,
                                         _c_int, _c_vp, _c_size, _c_vp, _c_vp, _c_vp,
                                         _c_vp]),
+    "ozk_matmul_flag_word": (_c_int, [_c_vp, _c_i64, _c_vp, _c_i64, _c_vp, _c_i64,
+                                      _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int,
+                                      _c_int, _c_vp, _c_size, _c_vp, _c_vp, _c_vp]),
+    "ozk_wait_flag_word": (_c_int, [_c_vp, _c_vp, ctypes.POINTER(ctypes.c_uint32)]),
     "ozk_matmul_noalloc": (_c_int, [_c_vp, _c_i64, _c_vp, _c_i64, _c_vp, _c_i64, _c_i64,
                                     _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_int,
                                     _c_vp, _c_vp]),
@@ -126,6 +130,8 @@ SIGNATURES = {
     "ozk_gram_early_flags": (_c_int, [_c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
                                       _c_vp, _c_i64, _c_vp, _c_size, _c_vp, _c_vp, _c_vp,
                                       _c_vp]),
+    "ozk_gram_flag_word": (_c_int, [_c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
+                                    _c_vp, _c_i64, _c_vp, _c_size, _c_vp, _c_vp, _c_vp]),
     "ozk_residual_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_i64, _c_int,
                                                _c_int]),
     "ozk_residual": (_c_int, [_c_vp, _c_i64, _c_vp, _c_i64, _c_vp, _c_i64, _c_vp,

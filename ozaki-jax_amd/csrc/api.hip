@@ -62,7 +62,7 @@ int launch_gemm(const void* As, const int32_t* Ae, const void* Bs,
                 const int32_t* Be, int64_t N, int64_t M, int64_t K, int pipe,
                 int nhi, int nlo, int order, double* C, int64_t ldc,
                 void* ws, size_t ws_bytes, hipStream_t st, bool i8, int rho,
-                const int32_t* Asum, const int32_t* Bsum);
+                const int32_t* Asum, const int32_t* Bsum, FlagPub pub = {});
 size_t gemm_workspace_bytes(int64_t N, int64_t M, int pipe, int nhi, int nlo,
                             int order);
 size_t gemm_state_bytes(int64_t N, int64_t M, int pipe, int nhi, int nlo, int order);
@@ -87,7 +87,7 @@ int launch_lu_solve(const float* LU, int64_t lda, const int32_t* perm, int64_t n
 bool gram_sym_supported(int nhi, int nlo);
 int launch_gram_sym(const void* S, const int32_t* E, int64_t n, int64_t K, int nhi,
                     int nlo, double* G, int64_t ldg, void* ws, size_t ws_bytes,
-                    hipStream_t st, bool i8, int rho, const int32_t* Ssum);
+                    hipStream_t st, bool i8, int rho, const int32_t* Ssum, FlagPub pub);
 size_t gemm_tail_bytes(int64_t N, int64_t M, int64_t K, int pipe, int nhi, int nlo,
                        bool sym, bool i8);
 bool residual_rows_supported(int64_t K, int64_t ncols, int nhi, int nlo);
@@ -492,11 +492,18 @@ static int flags_to_host(const uint32_t* flags, uint32_t* host_flags, void* even
   return OZK_OK;
 }
 
+// A call with no kernels, so with no flags.
+static int no_flags(const uint32_t* flags, uint32_t* host_flags, void* event, hipStream_t st,
+                    FlagPub pub) {
+  if (pub.host) *pub.host = OZK_FLAGS_READY;
+  return flags_to_host(flags, host_flags, event, st);
+}
+
 static int matmul_call(const double* A, int64_t lda, const double* B, int64_t ldb,
                        double* C, int64_t ldc, int64_t N, int64_t K, int64_t M,
                        int pipeline, int n_hi, int n_lo, int order, void* workspace,
                        size_t workspace_bytes, uint32_t* flags, uint32_t* host_flags,
-                       void* event, void* stream) {
+                       void* event, void* stream, FlagPub pub = {}) {
   clear_error();
   hipStream_t st = (hipStream_t)stream;
   const int pipe_arg = pipeline;
@@ -511,8 +518,8 @@ static int matmul_call(const double* A, int64_t lda, const double* B, int64_t ld
                     (ldc >= M || N <= 1),
                 "leading dimension smaller than the row length");
   OZK_CHECK_ARG(flags, "null flags pointer");
-  if ((rc = launch_fill_u32(flags, 0u, st))) return rc;
-  if (N == 0 || M == 0) return flags_to_host(flags, host_flags, event, st);
+  if (!pub.host && (rc = launch_fill_u32(flags, 0u, st))) return rc;
+  if (N == 0 || M == 0) return no_flags(flags, host_flags, event, st, pub);
   const size_t need = ozk_matmul_workspace_bytes(N, K, M, pipe_arg, n_hi, n_lo);
   if (!workspace || workspace_bytes < need) {
     set_error("matmul: workspace of %zu bytes needed, %zu given", need,
@@ -545,7 +552,7 @@ static int matmul_call(const double* A, int64_t lda, const double* B, int64_t ld
   }
   if ((rc = flags_to_host(flags, host_flags, event, st))) return rc;
   return launch_gemm(sa.s, sa.e, sb.s, sb.e, N, M, K, pipeline, n_hi, n_lo,
-                     order, C, ldc, gws, gwsb, st, i8, rho, sa.sum, sb.sum);
+                     order, C, ldc, gws, gwsb, st, i8, rho, sa.sum, sb.sum, pub);
 }
 
 int ozk_matmul(const double* A, int64_t lda, const double* B, int64_t ldb,
@@ -565,6 +572,50 @@ int ozk_matmul_early_flags(const double* A, int64_t lda, const double* B, int64_
   OZK_CHECK_ARG(host_flags && event, "null host flag word or event");
   return matmul_call(A, lda, B, ldb, C, ldc, N, K, M, pipeline, n_hi, n_lo, order,
                      workspace, workspace_bytes, flags, host_flags, event, stream);
+}
+
+int ozk_matmul_flag_word(const double* A, int64_t lda, const double* B, int64_t ldb,
+                         double* C, int64_t ldc, int64_t N, int64_t K, int64_t M,
+                         int pipeline, int n_hi, int n_lo, int order, void* workspace,
+                         size_t workspace_bytes, uint32_t* zero_flags, uint32_t* host_word,
+                         void* stream) {
+  clear_error();
+  OZK_CHECK_ARG(host_word, "null host flag word");
+  FlagPub pub;
+  pub.flags = zero_flags;
+  pub.host = host_word;
+  return matmul_call(A, lda, B, ldb, C, ldc, N, K, M, pipeline, n_hi, n_lo, order,
+                     workspace, workspace_bytes, zero_flags, nullptr, nullptr, stream, pub);
+}
+
+int ozk_wait_flag_word(const uint32_t* host_word, void* stream, uint32_t* flags) {
+  clear_error();
+  OZK_CHECK_ARG(host_word && flags, "null pointer");
+  hipStream_t st = (hipStream_t)stream;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  OZK_HIP(hipStreamIsCapturing(st, &cap));
+  if (cap != hipStreamCaptureStatusNone) {
+    set_error("the flags of a call under stream capture cannot be waited for");
+    return OZK_ERR_HIP;
+  }
+  // Between looks at the word the stream is asked for its state now and then:
+  // an error, or a drained stream whose word never came, ends the wait.
+  for (;;) {
+    for (int i = 0; i < 4096; ++i) {
+      const uint32_t v = __atomic_load_n(host_word, __ATOMIC_ACQUIRE);
+      if (v & OZK_FLAGS_READY) {
+        *flags = v & ~OZK_FLAGS_READY;
+        return OZK_OK;
+      }
+      __builtin_ia32_pause();
+    }
+    const hipError_t e = hipStreamQuery(st);
+    if (e == hipErrorNotReady) continue;
+    OZK_HIP(e);
+    if (__atomic_load_n(host_word, __ATOMIC_ACQUIRE) & OZK_FLAGS_READY) continue;
+    set_error("the stream is idle and the call's flags were never published");
+    return OZK_ERR_HIP;
+  }
 }
 
 static size_t gram_ws(int64_t rows, int64_t cols, int nhi, int nlo, void* ws,
@@ -596,7 +647,7 @@ size_t ozk_gram_workspace_bytes(int64_t rows, int64_t cols, int n_hi,
 static int gram_call(const double* A, int64_t lda, int64_t rows, int64_t cols, int n_hi,
                      int n_lo, double* G, int64_t ldg, void* workspace,
                      size_t workspace_bytes, uint32_t* flags, uint32_t* host_flags,
-                     void* event, void* stream) {
+                     void* event, void* stream, FlagPub pub = {}) {
   clear_error();
   hipStream_t st = (hipStream_t)stream;
   int rc = check_counts(OZK_PIPE_ONDEVICE, n_hi, n_lo);
@@ -606,8 +657,8 @@ static int gram_call(const double* A, int64_t lda, int64_t rows, int64_t cols, i
   OZK_CHECK_ARG((lda >= cols || rows <= 1) && (ldg >= cols || cols <= 1),
                 "leading dimension too small");
   OZK_CHECK_ARG(flags, "null flags pointer");
-  if ((rc = launch_fill_u32(flags, 0u, st))) return rc;
-  if (cols == 0) return flags_to_host(flags, host_flags, event, st);
+  if (!pub.host && (rc = launch_fill_u32(flags, 0u, st))) return rc;
+  if (cols == 0) return no_flags(flags, host_flags, event, st, pub);
   const size_t need = ozk_gram_workspace_bytes(rows, cols, n_hi, n_lo);
   if (!workspace || workspace_bytes < need) {
     set_error("gram: workspace of %zu bytes needed, %zu given", need,
@@ -631,10 +682,10 @@ static int gram_call(const double* A, int64_t lda, int64_t rows, int64_t cols, i
   // epilogue.  max (three K sweeps): full product, then symmetrise.
   if (gram_sym_supported(n_hi, n_lo))
     return launch_gram_sym(s.s, s.e, cols, rows, n_hi, n_lo, G, ldg, gws, gwsb, st, i8,
-                           rho, s.sum);
+                           rho, s.sum, pub);
   if ((rc = launch_gemm(s.s, s.e, s.s, s.e, cols, cols, rows, OZK_PIPE_ONDEVICE,
                         n_hi, n_lo, OZK_ORDER_2SUM, G, ldg, gws, gwsb, st, i8, rho, s.sum,
-                        s.sum)))
+                        s.sum, pub)))
     return rc;
   hipLaunchKernelGGL(symmetrize_kernel, dim3(grid_for(cols * cols)), dim3(256),
                      0, st, G, cols, ldg);
@@ -657,6 +708,19 @@ int ozk_gram_early_flags(const double* A, int64_t lda, int64_t rows, int64_t col
   OZK_CHECK_ARG(host_flags && event, "null host flag word or event");
   return gram_call(A, lda, rows, cols, n_hi, n_lo, G, ldg, workspace, workspace_bytes,
                    flags, host_flags, event, stream);
+}
+
+int ozk_gram_flag_word(const double* A, int64_t lda, int64_t rows, int64_t cols, int n_hi,
+                       int n_lo, double* G, int64_t ldg, void* workspace,
+                       size_t workspace_bytes, uint32_t* zero_flags, uint32_t* host_word,
+                       void* stream) {
+  clear_error();
+  OZK_CHECK_ARG(host_word, "null host flag word");
+  FlagPub pub;
+  pub.flags = zero_flags;
+  pub.host = host_word;
+  return gram_call(A, lda, rows, cols, n_hi, n_lo, G, ldg, workspace, workspace_bytes,
+                   zero_flags, nullptr, nullptr, stream, pub);
 }
 
 // Residual workspace.  Up to 4 right-hand sides with K <= 16384 (presets

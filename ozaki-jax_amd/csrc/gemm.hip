@@ -780,7 +780,7 @@ __global__ __launch_bounds__(kThreads16) void gemm_allpairs(
     int64_t N, int64_t M, int64_t nst, int64_t a_lines, int64_t b_lines,
     float unit2, double* __restrict__ C, int64_t ldc, float* __restrict__ P,
     int64_t ldp, char* __restrict__ state, int tail_P, uint32_t* __restrict__ part,
-    I8Fix fix, uint32_t* __restrict__ dyn, int dyn_nstat, int rflags) {
+    I8Fix fix, uint32_t* __restrict__ dyn, int dyn_nstat, int rflags, FlagPub pub) {
   typedef Sweep<PIPE, NHI, NLO, B0, B1, SYM> SW;
   constexpr int NA = SW::NA, NB = SW::NB, NP = SW::NP, RB = SW::RB, FA = SW::FA;
   constexpr int kBuf = SW::NFRAG * 64;  // uint4 per stage buffer
@@ -791,6 +791,8 @@ __global__ __launch_bounds__(kThreads16) void gemm_allpairs(
 
   const int ntm = (int)((a_lines + SW::TM - 1) / SW::TM), ntn = (int)(b_lines / kBN);
   const int bid = (int)blockIdx.x, nwg = (int)gridDim.x;
+  // (a wave that issues no stage loads)
+  if (pub.host && bid == 0 && threadIdx.x == 256) publish_flags(pub);
   // SYM: B's planes are A's (a gram matrix); only tiles tm <= tn are run
   // and each element folds both C[i][j] and C[j][i] (see the epilogue).
   static_assert(!SYM || (B0 == 0 && B1 == 2 && ORDER == OZK_ORDER_2SUM),
@@ -1179,6 +1181,8 @@ __global__ void probe_mfma16_kernel(int32_t* out) {
 
 // ---------------------------------------------------------------- launch
 
+__global__ void publish_flags_kernel(FlagPub pub) { publish_flags(pub); }
+
 __global__ void zero_u32_kernel(uint32_t* __restrict__ p, int n) {
   for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0u;
 }
@@ -1248,6 +1252,7 @@ struct ApArgs {
   int64_t ldp;
   char* state;
   I8Fix fix;
+  FlagPub pub;  // taken by the schedule's first sweep
 };
 
 // One sweep's kernel on operands As .. fix (the rectangle sweeps pass them
@@ -1285,7 +1290,7 @@ static void launch_sweep_kernel(const ApArgs& a, const char* As, const int32_t* 
   hipLaunchKernelGGL((gemm_allpairs<Op, PIPE, NHI, NLO, ORDER, B0, B1, SYM>), grid,
                      dim3(kThreads16), 0, a.st, As, Ae, Bs, Be, a.N, a.M, a.nst, a.al, a.bl,
                      a.unit2, a.C, a.ldc, a.P, a.ldp, a.state, tail_P, part, fix, dyn, nstat,
-                     rflags);
+                     rflags, SW::kFirst || (rflags & kRfFirst) ? a.pub : FlagPub{});
   if constexpr (SW::kFirst && SW::kLast) {
     if (tail_P > 1)
       hipLaunchKernelGGL((gemm_tail_fixup<Op, PIPE, NHI, NLO, ORDER, B0, B1, SYM>),
@@ -1657,7 +1662,7 @@ static int launch_allpairs(bool i8, int pipe, const void* As, const int32_t* Ae,
                            int order, double* C, int64_t ldc, float* P,
                            int64_t ldp, void* state, size_t state_bytes,
                            hipStream_t st, const int32_t* Asum, const int32_t* Bsum,
-                           bool sym = false) {
+                           bool sym = false, FlagPub pub = {}) {
   if (i8 && (!Asum || !Bsum)) {
     set_error("int8 slice planes need their line sums");
     return OZK_ERR_INVALID;
@@ -1703,6 +1708,7 @@ static int launch_allpairs(bool i8, int pipe, const void* As, const int32_t* Ae,
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, st, a.dyn, kDynSlot0);
   }
   a.sym = sym;
+  a.pub = pub;
   a.st = st;
   a.As = (const char*)As;
   a.Bs = (const char*)Bs;
@@ -1777,23 +1783,23 @@ bool gram_sym_supported(int nhi, int nlo) { return nlo == 1 && (nhi == 4 || nhi 
 
 int launch_gram_sym(const void* S, const int32_t* E, int64_t n, int64_t K, int nhi,
                     int nlo, double* G, int64_t ldg, void* ws, size_t ws_bytes,
-                    hipStream_t st, bool i8, int rho, const int32_t* Ssum) {
+                    hipStream_t st, bool i8, int rho, const int32_t* Ssum, FlagPub pub) {
   if (!gram_sym_supported(nhi, nlo)) {
     set_error("symmetric gram needs the high or medium preset");
     return OZK_ERR_UNSUPPORTED;
   }
   return launch_allpairs(i8, OZK_PIPE_ONDEVICE, S, E, S, E, n, n, K, rho, nhi, nlo, OZK_ORDER_2SUM, G, ldg,
-                         nullptr, 0, ws, ws_bytes, st, Ssum, Ssum, true);
+                         nullptr, 0, ws, ws_bytes, st, Ssum, Ssum, true, pub);
 }
 
 int launch_gemm(const void* As, const int32_t* Ae, const void* Bs,
                 const int32_t* Be, int64_t N, int64_t M, int64_t K, int pipe,
                 int nhi, int nlo, int order, double* C, int64_t ldc,
                 void* ws, size_t ws_bytes, hipStream_t st, bool i8, int rho,
-                const int32_t* Asum, const int32_t* Bsum) {
+                const int32_t* Asum, const int32_t* Bsum, FlagPub pub) {
   if (allpairs_schedule(pipe, nhi, nlo) && allpairs_order(pipe, nhi, nlo, order))
     return launch_allpairs(i8, pipe, As, Ae, Bs, Be, N, M, K, rho, nhi, nlo, order,
-                           C, ldc, nullptr, 0, ws, ws_bytes, st, Asum, Bsum);
+                           C, ldc, nullptr, 0, ws, ws_bytes, st, Asum, Bsum, false, pub);
   if (i8) {
     set_error("int8 slice planes need an all-pairs on-device schedule");
     return OZK_ERR_UNSUPPORTED;
@@ -1805,6 +1811,10 @@ int launch_gemm(const void* As, const int32_t* Ae, const void* Bs,
   const dim3 grid((unsigned)ntiles);
   const uint16_t* A16 = (const uint16_t*)As;
   const uint16_t* B16 = (const uint16_t*)Bs;
+  if (pub.host) {
+    hipLaunchKernelGGL(publish_flags_kernel, dim3(1), dim3(1), 0, st, pub);
+    OZK_LAUNCH_CHECK();
+  }
 #define OZK_PW(O)                                                              \
   hipLaunchKernelGGL((gemm_pairwise<O, 0>), grid, dim3(kThreads), 0, st, A16,  \
                      Ae, B16, Be, N, M, ld, al, bl, pipe, nhi, nlo, C, ldc,    \

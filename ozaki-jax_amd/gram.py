@@ -44,22 +44,16 @@ def gram(A, precision="high", accumulation="bf16_interleaved", mode="f64"):
     # A NaN / Inf in A gives NaN rows and columns of G, as in the reference,
     # which runs no preflight here; the flag word is read only for
     # OZK_FLAG_WAIT_TIMEOUT.
-    flags = fam.flags()
-    early = getattr(fam, "early_flags", None)
 
     def once():
+        # read once the extraction has run; G is returned while the GEMM is
+        # still queued on the stream
         wsb = lib.ozk_gram_workspace_bytes(rows, cols, n_hi, n_lo)
         ws = fam.workspace(wsb)
-        args = (At.data_ptr(), D.ld_of(At), rows, cols, n_hi, n_lo, G.data_ptr(),
-                D.ld_of(G), ws.data_ptr(), wsb, flags.data_ptr())
-        if early is None:
-            _lib.check(lib.ozk_gram(*args, fam.stream()))
-            return fam.read_flags(flags)
-        # torch tensors: the flags are read once the extraction has run; G is
-        # returned while the GEMM is still queued on the current stream
-        word, ev, read = early()
-        _lib.check(lib.ozk_gram_early_flags(*args, word, ev, fam.stream()))
-        return read()
+        stream = fam.stream()
+        return fam.flag_words().run(lambda flags, word: lib.ozk_gram_flag_word(
+            At.data_ptr(), D.ld_of(At), rows, cols, n_hi, n_lo, G.data_ptr(),
+            D.ld_of(G), ws.data_ptr(), wsb, flags, word, stream), stream)
 
     _lib.with_gang_retry(once)
     return fam.out(G, want_torch)

@@ -121,23 +121,17 @@ def _run_matmul(fam, At, Bt, pipeline, n_hi, n_lo, order):
     C = fam.empty((N, M))
     if N == 0 or M == 0:
         return C, 0
-    flags = fam.flags()  # cleared by the call
-    early = getattr(fam, "early_flags", None)
 
     def once(pipe):
+        # the flags are read once the extraction has run; C is returned while
+        # the GEMM is still queued on the stream
         wsb = lib.ozk_matmul_workspace_bytes(N, K, M, pipe, n_hi, n_lo)
         ws = fam.workspace(wsb)
-        args = (At.data_ptr(), D.ld_of(At), Bt.data_ptr(), D.ld_of(Bt), C.data_ptr(),
-                D.ld_of(C), N, K, M, pipe, n_hi, n_lo, order, ws.data_ptr(), wsb,
-                flags.data_ptr())
-        if early is None:
-            _lib.check(lib.ozk_matmul(*args, fam.stream()))
-            return fam.read_flags(flags)
-        # torch tensors: the flags are read once the extraction has run, and
-        # C is returned while the GEMM is still queued on the current stream
-        word, ev, read = early()
-        _lib.check(lib.ozk_matmul_early_flags(*args, word, ev, fam.stream()))
-        return read()
+        stream = fam.stream()
+        return fam.flag_words().run(lambda flags, word: lib.ozk_matmul_flag_word(
+            At.data_ptr(), D.ld_of(At), Bt.data_ptr(), D.ld_of(Bt), C.data_ptr(),
+            D.ld_of(C), N, K, M, pipe, n_hi, n_lo, order, ws.data_ptr(), wsb,
+            flags, word, stream), stream)
 
     def run(pipe):
         return _lib.with_gang_retry(lambda: once(pipe))
