@@ -51,7 +51,9 @@ template <typename W>
 int extract(const double* X, int64_t rows, int64_t cols, int64_t ldx,
             int by_cols, int rho, int n0, int n1, void* S, int32_t* E,
             uint32_t* flags, void* ws, size_t wsb, hipStream_t st, bool i8,
-            int32_t* sums);
+            int32_t* sums, ZeroJobs zero = {}, bool zeroed = false);
+bool column_zero_jobs(int64_t arows, int64_t acols, int64_t rows, int64_t cols, int n0, int n1,
+                      void* ws, int32_t* Sg, ZeroJobs& z);
 size_t extract_workspace_bytes(int64_t rows, int64_t cols, int by_cols, bool f64);
 int launch_fill_u32(uint32_t* p, uint32_t v, hipStream_t st);
 int launch_check_finite(const double* X, int64_t rows, int64_t cols,
@@ -62,7 +64,10 @@ int launch_gemm(const void* As, const int32_t* Ae, const void* Bs,
                 const int32_t* Be, int64_t N, int64_t M, int64_t K, int pipe,
                 int nhi, int nlo, int order, double* C, int64_t ldc,
                 void* ws, size_t ws_bytes, hipStream_t st, bool i8, int rho,
-                const int32_t* Asum, const int32_t* Bsum, FlagPub pub = {});
+                const int32_t* Asum, const int32_t* Bsum, FlagPub pub = {},
+                bool dyn_zeroed = false);
+size_t gemm_dyn_counters(int64_t N, int64_t M, int pipe, int nhi, int nlo, int order,
+                         size_t* bytes);
 size_t gemm_workspace_bytes(int64_t N, int64_t M, int pipe, int nhi, int nlo,
                             int order);
 size_t gemm_state_bytes(int64_t N, int64_t M, int pipe, int nhi, int nlo, int order);
@@ -87,7 +92,8 @@ int launch_lu_solve(const float* LU, int64_t lda, const int32_t* perm, int64_t n
 bool gram_sym_supported(int nhi, int nlo);
 int launch_gram_sym(const void* S, const int32_t* E, int64_t n, int64_t K, int nhi,
                     int nlo, double* G, int64_t ldg, void* ws, size_t ws_bytes,
-                    hipStream_t st, bool i8, int rho, const int32_t* Ssum, FlagPub pub);
+                    hipStream_t st, bool i8, int rho, const int32_t* Ssum, FlagPub pub,
+                    bool dyn_zeroed);
 size_t gemm_tail_bytes(int64_t N, int64_t M, int64_t K, int pipe, int nhi, int nlo,
                        bool sym, bool i8);
 bool residual_rows_supported(int64_t K, int64_t ncols, int nhi, int nlo);
@@ -533,18 +539,24 @@ static int matmul_call(const double* A, int64_t lda, const double* B, int64_t ld
             &gwsb);
   const size_t tbytes = extract_pair_bytes(N, K, M, pipeline != OZK_PIPE_ONDEVICE);
   int rho;
+  // A's extraction clears what B's and the GEMM need at zero
+  ZeroJobs zero;
+  size_t dyn_bytes;
+  const size_t dyn_off = gemm_dyn_counters(N, M, pipeline, n_hi, n_lo, order, &dyn_bytes);
+  zero.add((char*)gws + dyn_off, dyn_bytes);
   if (pipeline == OZK_PIPE_ONDEVICE) {
     rho = rho_generic(K, 24);
+    const bool zeroed = column_zero_jobs(N, K, K, M, n_hi, n_lo, tws, sb.sum, zero);
     if ((rc = extract<float>(A, N, K, lda, 0, rho, n_hi, n_lo, sa.s, sa.e, flags,
-                             tws, tbytes, st, i8, sa.sum)))
+                             tws, tbytes, st, i8, sa.sum, zero)))
       return rc;
     if ((rc = extract<float>(B, K, M, ldb, 1, rho, n_hi, n_lo, sb.s, sb.e, flags,
-                             tws, tbytes, st, i8, sb.sum)))
+                             tws, tbytes, st, i8, sb.sum, {}, zeroed)))
       return rc;
   } else {
     rho = rho_generic(K, 53);
     if ((rc = extract<double>(A, N, K, lda, 0, rho, n_hi, 0, sa.s, sa.e, flags,
-                              tws, tbytes, st, false, nullptr)))
+                              tws, tbytes, st, false, nullptr, zero)))
       return rc;
     if ((rc = extract<double>(B, K, M, ldb, 1, rho, n_hi, 0, sb.s, sb.e, flags,
                               tws, tbytes, st, false, nullptr)))
@@ -552,7 +564,7 @@ static int matmul_call(const double* A, int64_t lda, const double* B, int64_t ld
   }
   if ((rc = flags_to_host(flags, host_flags, event, st))) return rc;
   return launch_gemm(sa.s, sa.e, sb.s, sb.e, N, M, K, pipeline, n_hi, n_lo,
-                     order, C, ldc, gws, gwsb, st, i8, rho, sa.sum, sb.sum, pub);
+                     order, C, ldc, gws, gwsb, st, i8, rho, sa.sum, sb.sum, pub, true);
 }
 
 int ozk_matmul(const double* A, int64_t lda, const double* B, int64_t ldb,
@@ -673,19 +685,24 @@ static int gram_call(const double* A, int64_t lda, int64_t rows, int64_t cols, i
   // both operands (gram.py:22-35 extracts the same values twice).
   const int rho = rho_generic(rows, 24);
   const bool i8 = use_i8(OZK_PIPE_ONDEVICE, rows, n_hi, n_lo);
+  ZeroJobs zero;
+  size_t dyn_bytes;
+  const size_t dyn_off =
+      gemm_dyn_counters(cols, cols, OZK_PIPE_ONDEVICE, n_hi, n_lo, OZK_ORDER_2SUM, &dyn_bytes);
+  zero.add((char*)gws + dyn_off, dyn_bytes);
   if ((rc = extract<float>(A, rows, cols, lda, 1, rho, n_hi, n_lo, s.s, s.e,
                            flags, tws, extract_workspace_bytes(rows, cols, 1, false), st,
-                           i8, s.sum)))
+                           i8, s.sum, zero)))
     return rc;
   if ((rc = flags_to_host(flags, host_flags, event, st))) return rc;
   // high / medium: upper tiles only, the symmetrisation folded into the
   // epilogue.  max (three K sweeps): full product, then symmetrise.
   if (gram_sym_supported(n_hi, n_lo))
     return launch_gram_sym(s.s, s.e, cols, rows, n_hi, n_lo, G, ldg, gws, gwsb, st, i8,
-                           rho, s.sum, pub);
+                           rho, s.sum, pub, true);
   if ((rc = launch_gemm(s.s, s.e, s.s, s.e, cols, cols, rows, OZK_PIPE_ONDEVICE,
                         n_hi, n_lo, OZK_ORDER_2SUM, G, ldg, gws, gwsb, st, i8, rho, s.sum,
-                        s.sum, pub)))
+                        s.sum, pub, true)))
     return rc;
   hipLaunchKernelGGL(symmetrize_kernel, dim3(grid_for(cols * cols)), dim3(256),
                      0, st, G, cols, ldg);

@@ -82,6 +82,34 @@ __device__ __forceinline__ void publish_flags(FlagPub pub) {
   __hip_atomic_store(pub.host, f | OZK_FLAGS_READY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Regions that later kernels of a call need at zero, cleared by workgroups
+// appended to an extraction kernel that runs before them (or by one launch
+// where there is none): a launch of its own for each cost about 5 us on a busy
+// stream.  Sizes in 16-byte units.
+struct ZeroJobs {
+  uint4* p[4] = {};
+  int64_t n[4] = {};
+  int count = 0;
+  void add(void* q, size_t bytes) {
+    if (!q || bytes == 0) return;
+    p[count] = (uint4*)q;
+    n[count++] = (int64_t)(bytes / 16);
+  }
+  int64_t units() const { return n[0] + n[1] + n[2] + n[3]; }
+  // workgroups of `threads` threads for them: up to eight stores a thread
+  int64_t groups(int threads) const {
+    const int64_t g = (units() + threads * 8 - 1) / (threads * 8);
+    return g < 1024 ? g : 1024;
+  }
+};
+
+// Workgroup `g` of `ng` with the jobs.
+__device__ __forceinline__ void run_zero_jobs(const ZeroJobs& z, int64_t g, int64_t ng) {
+  for (int j = 0; j < z.count; ++j)
+    for (int64_t i = g * blockDim.x + threadIdx.x; i < z.n[j]; i += ng * blockDim.x)
+      z.p[j][i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 // ---------------------------------------------------------------- layout
 // Slice planes hold BF16 bit patterns or INT8 grid counts with lines padded
 // to kLinePad and k padded to kKPad elements; padding holds zeros, so the

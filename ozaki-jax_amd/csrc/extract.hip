@@ -200,7 +200,11 @@ __global__ __launch_bounds__(BLOCK * LPB) void extract_lines_reg(
     const double* __restrict__ X, int64_t lines, int64_t len, int64_t ldx,
     int vec_ok, int rho, int n0, int n1, typename PlaneElem<FMT>::type* __restrict__ S,
     int64_t ld, int64_t plane, int32_t* __restrict__ E, int64_t eplane,
-    uint32_t* __restrict__ flags, int32_t* __restrict__ Sg) {
+    uint32_t* __restrict__ flags, int32_t* __restrict__ Sg, int ngroups, ZeroJobs zero) {
+  if ((int)blockIdx.x >= ngroups) {  // behind the lines' workgroups
+    run_zero_jobs(zero, (int)blockIdx.x - ngroups, (int)gridDim.x - ngroups);
+    return;
+  }
   static_assert(VEC == 2 || VEC == 4, "VEC doubles are read as 16-byte pairs");
   const float qscale = ldexpf(1.0f, 24 - rho);
   constexpr int NP = Parts<W>::N;
@@ -213,7 +217,7 @@ __global__ __launch_bounds__(BLOCK * LPB) void extract_lines_reg(
     for (int i = threadIdx.x; i < kMaxPlanes * LPB; i += BLOCK * LPB) ssum[i] = 0;
   }
   const int t = threadIdx.x % BLOCK;
-  const int64_t grp = xcd_line(blockIdx.x, gridDim.x);
+  const int64_t grp = xcd_line(blockIdx.x, ngroups);
   const int64_t line = grp * LPB + threadIdx.x / BLOCK;
   const bool live = line < lines;
   // Plane offset of the thread's first element: BLOCK * VEC is a multiple of
@@ -909,7 +913,11 @@ __global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(4
     const double* __restrict__ X, int64_t K, int64_t M, int64_t ldx, int rho, int n0, int n1,
     typename PlaneElem<FMT>::type* __restrict__ S, int64_t ld, int64_t plane,
     int32_t* __restrict__ E, int64_t eplane, uint32_t* __restrict__ flags,
-    int32_t* __restrict__ Sg) {
+    int32_t* __restrict__ Sg, int npanels, ZeroJobs zero) {
+  if ((int)blockIdx.x >= npanels) {  // behind the panels' workgroups
+    run_zero_jobs(zero, (int)blockIdx.x - npanels, (int)gridDim.x - npanels);
+    return;
+  }
   typedef typename PlaneElem<FMT>::type T;
   constexpr int NP = 2, NW = kPanelThreads / 64;
   constexpr int BYTES = RPT * (int)sizeof(T);  // plane bytes of a thread's rows
@@ -921,7 +929,7 @@ __global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(4
   if constexpr (FMT == kFmtI8) {
     for (int i = t; i < kMaxPlanes * kPanelCols; i += kPanelThreads) ssum[i] = 0;
   }
-  const int64_t panel = xcd_line(blockIdx.x, gridDim.x);
+  const int64_t panel = xcd_line(blockIdx.x, npanels);
   const int cl = t % kPanelCols;
   const int64_t line = panel * kPanelCols + cl;  // the thread's column
   const int64_t r0 = (int64_t)RPT * (t / kPanelCols);
@@ -1218,17 +1226,7 @@ __global__ __launch_bounds__(kRowThreads) void extract_lines_gang(
   }
 }
 
-__global__ void zero_i32_kernel(int32_t* __restrict__ p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = 0;
-}
-
-__global__ void zero_u32x4_kernel(uint4* __restrict__ p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = make_uint4(0u, 0u, 0u, 0u);
-}
+__global__ void zero_jobs_kernel(ZeroJobs z) { run_zero_jobs(z, blockIdx.x, gridDim.x); }
 
 // X (rows x cols, ldx) -> XT (cols x rows, contiguous) through LDS tiles of
 // 128 rows x 64 columns: each wave reads 512 contiguous bytes of a row of X
@@ -1330,10 +1328,18 @@ static size_t row_gang_bytes(int64_t lines, int64_t, int nslices) {
   return (size_t)round_up(kGangHeader + round_up(lines, kLinePad) * nslices * kRowRecBytes, 256);
 }
 
+// One launch for the jobs.
+static int launch_zero_jobs(const ZeroJobs& z, hipStream_t st) {
+  if (z.units() == 0) return OZK_OK;
+  hipLaunchKernelGGL(zero_jobs_kernel, dim3((unsigned)z.groups(256)), dim3(256), 0, st, z);
+  OZK_LAUNCH_CHECK();
+  return OZK_OK;
+}
+
 template <int FMT>
 static int launch_rows_gang(const double* X, int64_t lines, int64_t len, int64_t ldx,
                             int rho, int n0, int n1, void* Sv, int32_t* E, uint32_t* flags,
-                            void* ws, size_t wsb, hipStream_t st, int32_t* Sg) {
+                            void* ws, size_t wsb, hipStream_t st, int32_t* Sg, ZeroJobs zero) {
   typedef typename PlaneElem<FMT>::type T;
   const int ns = n0 > n1 ? n0 : n1;
   const size_t need = row_gang_bytes(lines, len, ns);
@@ -1345,17 +1351,10 @@ static int launch_rows_gang(const double* X, int64_t lines, int64_t len, int64_t
   const int64_t plane = lp * ld;
   const int G = (int)((ld + kRowRun - 1) / kRowRun);
   // the ticket, the exchange records and the INT8 line sums start at zero
-  const int64_t n16 = (int64_t)need / 16;
-  hipLaunchKernelGGL(zero_u32x4_kernel,
-                     dim3((unsigned)((n16 + 255) / 256 < 1024 ? (n16 + 255) / 256 : 1024)),
-                     dim3(256), 0, st, (uint4*)ws, n16);
-  OZK_LAUNCH_CHECK();
-  if constexpr (FMT == kFmtI8) {
-    const int64_t ns32 = (int64_t)(n0 + n1) * lp;
-    hipLaunchKernelGGL(zero_i32_kernel, dim3((unsigned)((ns32 + 255) / 256 < 1024 ? (ns32 + 255) / 256 : 1024)),
-                       dim3(256), 0, st, Sg, ns32);
-    OZK_LAUNCH_CHECK();
-  }
+  zero.add(ws, need);
+  if (FMT == kFmtI8) zero.add(Sg, (size_t)(n0 + n1) * lp * sizeof(int32_t));
+  const int rc = launch_zero_jobs(zero, st);
+  if (rc) return rc;
   uint32_t* ticket = (uint32_t*)ws;
   uint32_t* rec = (uint32_t*)((char*)ws + kGangHeader);
   const dim3 grid((unsigned)(lp * G));
@@ -1376,11 +1375,11 @@ template <typename W, int FMT>
 static int launch_lines(const double* X, int64_t lines, int64_t len,
                         int64_t ldx, int rho, int n0, int n1, void* Sv,
                         int32_t* E, uint32_t* flags, void* ws, size_t wsb, hipStream_t st,
-                        int32_t* Sg) {
+                        int32_t* Sg, const ZeroJobs& zero) {
   if constexpr (sizeof(W) == 4) {
     if (gang_rows(len) && lines > 0)
       return launch_rows_gang<FMT>(X, lines, len, ldx, rho, n0, n1, Sv, E, flags, ws, wsb,
-                                   st, Sg);
+                                   st, Sg, zero);
   }
   typedef typename PlaneElem<FMT>::type T;
   T* S = (T*)Sv;
@@ -1392,8 +1391,9 @@ static int launch_lines(const double* X, int64_t lines, int64_t len,
   const int vec_ok = ((uintptr_t)X % 16 == 0) && (ldx % 2 == 0);
 #define OZK_REG(B, EPT, LPB, V)                                                        \
   hipLaunchKernelGGL((extract_lines_reg<W, B, EPT, LPB, FMT, V>),                      \
-                     dim3((unsigned)(lp / LPB)), dim3(B * LPB), 0, st, X, lines, len, ldx, \
-                     vec_ok && len % V == 0, rho, n0, n1, S, ld, plane, E, lp, flags, Sg)
+                     dim3((unsigned)(lp / LPB + zero.groups(B * LPB))), dim3(B * LPB), 0, st, \
+                     X, lines, len, ldx, vec_ok && len % V == 0, rho, n0, n1, S, ld, plane, \
+                     E, lp, flags, Sg, (int)(lp / LPB), zero)
   // Shapes measured per line-length bucket (one or two lines per workgroup
   // so that several workgroups share a CU and overlap loads with stores).
   if (ld <= 256) {
@@ -1417,6 +1417,8 @@ static int launch_lines(const double* X, int64_t lines, int64_t len,
       }
     }
     if (!done) {  // FP64 lines, and FP32 lines longer than the row gangs take
+      const int rc = launch_zero_jobs(zero, st);
+      if (rc) return rc;
       hipLaunchKernelGGL((extract_lines_stream<W, 1024, FMT>), grid, dim3(1024),
                          0, st, X, lines, len, ldx, rho, n0, n1, S, ld, plane, E,
                          lp, flags);
@@ -1458,15 +1460,17 @@ static bool panel_columns(int64_t rows) {
 template <int FMT>
 static int launch_cols_panel(const double* X, int64_t rows, int64_t cols, int64_t ldx,
                              int rho, int n0, int n1, void* Sv, int32_t* E, uint32_t* flags,
-                             hipStream_t st, int32_t* Sg) {
+                             hipStream_t st, int32_t* Sg, const ZeroJobs& zero) {
   typedef typename PlaneElem<FMT>::type T;
   if (rows <= 0 || cols <= 0) return OZK_OK;
   const int64_t ld = round_up(rows, kKPad), lp = round_up(cols, kLinePad);
   const int64_t plane = lp * ld;
-  const dim3 grid((unsigned)(lp / kPanelCols));
+  const int npanels = (int)(lp / kPanelCols);
+  const dim3 grid((unsigned)(npanels + zero.groups(kPanelThreads)));
 #define OZK_PANEL_LAUNCH(RPT)                                                              \
   hipLaunchKernelGGL((extract_cols_panel<FMT, RPT>), grid, dim3(kPanelThreads), 0, st, X,  \
-                     rows, cols, ldx, rho, n0, n1, (T*)Sv, ld, plane, E, lp, flags, Sg)
+                     rows, cols, ldx, rho, n0, n1, (T*)Sv, ld, plane, E, lp, flags, Sg,    \
+                     npanels, zero)
   if (ld <= kPanelGroups * 4)
     OZK_PANEL_LAUNCH(4);
   else if (ld <= kPanelGroups * 8)
@@ -1499,10 +1503,29 @@ size_t extract_workspace_bytes(int64_t rows, int64_t cols, int by_cols, bool f64
          (!f64 && gang_rows(rows) ? row_gang_bytes(cols, rows, kMaxSlices) : 0);
 }
 
+// What a column gang extraction needs at zero.
+static void add_gang_jobs(ZeroJobs& z, int64_t rows, int64_t cols, int n0, int n1, void* ws,
+                          int32_t* Sg) {
+  z.add(ws, gang_workspace_bytes(rows, cols, n0 > n1 ? n0 : n1));
+  z.add(Sg, (size_t)(n0 + n1) * round_up(cols, kLinePad) * sizeof(int32_t));
+}
+
+// Regions that an FP32 column extraction needs at zero (none but for the gangs):
+// `extract` of its rows' operand may clear them, and extract(.., zeroed =
+// true) then does not.  False when that extraction clears a workspace of its
+// own, which the two share.
+bool column_zero_jobs(int64_t arows, int64_t acols, int64_t rows, int64_t cols, int n0, int n1,
+                      void* ws, int32_t* Sg, ZeroJobs& z) {
+  if (panel_columns(rows) || !gang_columns(rows) || (gang_rows(acols) && arows > 0)) return false;
+  add_gang_jobs(z, rows, cols, n0, n1, ws, Sg);
+  return true;
+}
+
 template <int FMT>
 static int launch_cols_gang(const double* X, int64_t rows, int64_t cols, int64_t ldx,
                             int rho, int n0, int n1, void* Sv, int32_t* E, uint32_t* flags,
-                            void* ws, size_t wsb, hipStream_t st, int32_t* Sg) {
+                            void* ws, size_t wsb, hipStream_t st, int32_t* Sg, ZeroJobs zero,
+                            bool zeroed) {
   typedef typename PlaneElem<FMT>::type T;
   if (rows <= 0 || cols <= 0) return OZK_OK;
   const int ns = n0 > n1 ? n0 : n1;
@@ -1515,16 +1538,10 @@ static int launch_cols_gang(const double* X, int64_t rows, int64_t cols, int64_t
   const int64_t plane = lp * ld, npanels = lp / kGangPW;
   const int G = gang_members(ld);
   // the ticket, the exchange records and the INT8 line sums start at zero
-  const int64_t n16 = (int64_t)need / 16;
-  hipLaunchKernelGGL(zero_u32x4_kernel, dim3((unsigned)((n16 + 255) / 256 < 1024 ? (n16 + 255) / 256 : 1024)),
-                     dim3(256), 0, st, (uint4*)ws, n16);
-  OZK_LAUNCH_CHECK();
-  if constexpr (FMT == kFmtI8) {
-    const int64_t ns32 = (int64_t)(n0 + n1) * lp;
-    hipLaunchKernelGGL(zero_i32_kernel, dim3((unsigned)((ns32 + 255) / 256 < 1024 ? (ns32 + 255) / 256 : 1024)),
-                       dim3(256), 0, st, Sg, ns32);
-    OZK_LAUNCH_CHECK();
-  }
+  if (!zeroed)
+    add_gang_jobs(zero, rows, cols, n0, n1, ws, FMT == kFmtI8 ? Sg : nullptr);
+  const int rc = launch_zero_jobs(zero, st);
+  if (rc) return rc;
   uint32_t* ticket = (uint32_t*)ws;
   uint32_t* rec = (uint32_t*)((char*)ws + kGangHeader);
   const dim3 grid((unsigned)(npanels * G));
@@ -1544,7 +1561,7 @@ template <typename W>
 int extract(const double* X, int64_t rows, int64_t cols, int64_t ldx,
             int by_cols, int rho, int n0, int n1, void* S, int32_t* E,
             uint32_t* flags, void* ws, size_t wsb, hipStream_t st, bool i8,
-            int32_t* sums) {
+            int32_t* sums, ZeroJobs zero, bool zeroed) {
   if (i8 && (sizeof(W) != 4 || rho < 19 || rho > 24)) {
     set_error("int8 slice planes need the FP32 path with 19 <= rho <= 24 (rho=%d)", rho);
     return OZK_ERR_UNSUPPORTED;
@@ -1559,16 +1576,16 @@ int extract(const double* X, int64_t rows, int64_t cols, int64_t ldx,
     if (by_cols && panel_columns(rows)) {
       if (i8)
         return launch_cols_panel<kFmtI8>(X, rows, cols, ldx, rho, n0, n1, S, E, flags, st,
-                                         sums);
+                                         sums, zero);
       return launch_cols_panel<kFmtBf16>(X, rows, cols, ldx, rho, n0, n1, S, E, flags, st,
-                                         nullptr);
+                                         nullptr, zero);
     }
     if (by_cols && gang_columns(rows)) {
       if (i8)
         return launch_cols_gang<kFmtI8>(X, rows, cols, ldx, rho, n0, n1, S, E, flags, ws,
-                                        wsb, st, sums);
+                                        wsb, st, sums, zero, zeroed);
       return launch_cols_gang<kFmtBf16>(X, rows, cols, ldx, rho, n0, n1, S, E, flags, ws,
-                                        wsb, st, nullptr);
+                                        wsb, st, nullptr, zero, zeroed);
     }
   }
   if (by_cols) {
@@ -1591,17 +1608,17 @@ int extract(const double* X, int64_t rows, int64_t cols, int64_t ldx,
   }
   if (i8)
     return launch_lines<W, kFmtI8>(src, lines, len, lds, rho, n0, n1, S, E, flags, ws, wsb, st,
-                                   sums);
+                                   sums, zero);
   return launch_lines<W, kFmtBf16>(src, lines, len, lds, rho, n0, n1, S, E, flags, ws, wsb,
-                                   st, nullptr);
+                                   st, nullptr, zero);
 }
 
 template int extract<float>(const double*, int64_t, int64_t, int64_t, int, int,
                             int, int, void*, int32_t*, uint32_t*, void*,
-                            size_t, hipStream_t, bool, int32_t*);
+                            size_t, hipStream_t, bool, int32_t*, ZeroJobs, bool);
 template int extract<double>(const double*, int64_t, int64_t, int64_t, int, int,
                              int, int, void*, int32_t*, uint32_t*, void*,
-                             size_t, hipStream_t, bool, int32_t*);
+                             size_t, hipStream_t, bool, int32_t*, ZeroJobs, bool);
 
 int launch_check_finite(const double* X, int64_t rows, int64_t cols,
                         int64_t ld, uint32_t* flags, hipStream_t st) {

@@ -791,8 +791,11 @@ __global__ __launch_bounds__(kThreads16) void gemm_allpairs(
 
   const int ntm = (int)((a_lines + SW::TM - 1) / SW::TM), ntn = (int)(b_lines / kBN);
   const int bid = (int)blockIdx.x, nwg = (int)gridDim.x;
-  // (a wave that issues no stage loads)
-  if (pub.host && bid == 0 && threadIdx.x == 256) publish_flags(pub);
+  // (a wave that issues no stage loads; the symmetric form, whose scalar
+  // registers are short, ran 1.2% slower with this and takes
+  // publish_flags_kernel)
+  if constexpr (!SYM)
+    if (pub.host && bid == 0 && threadIdx.x == 256) publish_flags(pub);
   // SYM: B's planes are A's (a gram matrix); only tiles tm <= tn are run
   // and each element folds both C[i][j] and C[j][i] (see the epilogue).
   static_assert(!SYM || (B0 == 0 && B1 == 2 && ORDER == OZK_ORDER_2SUM),
@@ -1626,6 +1629,17 @@ size_t gemm_workspace_bytes(int64_t N, int64_t M, int pipe, int nhi, int nlo,
          kDynBytes;
 }
 
+// The dynamic-tail counters inside a workspace of gemm_workspace_bytes(), which
+// launch_gemm and launch_gram_sym (dyn_zeroed) let the caller clear: their
+// byte offset, and their bytes (0: the schedule has none).
+size_t gemm_dyn_counters(int64_t N, int64_t M, int pipe, int nhi, int nlo, int order,
+                         size_t* bytes) {
+  *bytes = 0;
+  if (!allpairs_schedule(pipe, nhi, nlo) || !allpairs_order(pipe, nhi, nlo, order)) return 0;
+  *bytes = kDynSlot0 * sizeof(uint32_t);
+  return (size_t)round_up((int64_t)gemm_state_bytes(N, M, pipe, nhi, nlo, order), 256);
+}
+
 // Tile rows of the all-pairs launch of schedule (nhi, nlo): those of its
 // single sweep; 64 for a multi-sweep schedule, whose sweeps size their own
 // grids (64-row tiles give the most tiles, the bound the launch checks).
@@ -1662,7 +1676,7 @@ static int launch_allpairs(bool i8, int pipe, const void* As, const int32_t* Ae,
                            int order, double* C, int64_t ldc, float* P,
                            int64_t ldp, void* state, size_t state_bytes,
                            hipStream_t st, const int32_t* Asum, const int32_t* Bsum,
-                           bool sym = false, FlagPub pub = {}) {
+                           bool sym = false, FlagPub pub = {}, bool dyn_zeroed = false) {
   if (i8 && (!Asum || !Bsum)) {
     set_error("int8 slice planes need their line sums");
     return OZK_ERR_INVALID;
@@ -1705,10 +1719,13 @@ static int launch_allpairs(bool i8, int pipe, const void* As, const int32_t* Ae,
       (allpairs_sweeps(pipe, nhi, nlo) > 1 ||
        dyn_static_rounds(ntiles, (int)a.grid.x, allpairs_nst(K, i8)) > 0)) {
     a.dyn = (uint32_t*)((char*)state + off);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, st, a.dyn, kDynSlot0);
+    if (!dyn_zeroed)
+      hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, st, a.dyn, kDynSlot0);
   }
   a.sym = sym;
   a.pub = pub;
+  if (sym && pub.host)
+    hipLaunchKernelGGL(publish_flags_kernel, dim3(1), dim3(1), 0, st, pub);
   a.st = st;
   a.As = (const char*)As;
   a.Bs = (const char*)Bs;
@@ -1783,23 +1800,25 @@ bool gram_sym_supported(int nhi, int nlo) { return nlo == 1 && (nhi == 4 || nhi 
 
 int launch_gram_sym(const void* S, const int32_t* E, int64_t n, int64_t K, int nhi,
                     int nlo, double* G, int64_t ldg, void* ws, size_t ws_bytes,
-                    hipStream_t st, bool i8, int rho, const int32_t* Ssum, FlagPub pub) {
+                    hipStream_t st, bool i8, int rho, const int32_t* Ssum, FlagPub pub,
+                    bool dyn_zeroed) {
   if (!gram_sym_supported(nhi, nlo)) {
     set_error("symmetric gram needs the high or medium preset");
     return OZK_ERR_UNSUPPORTED;
   }
   return launch_allpairs(i8, OZK_PIPE_ONDEVICE, S, E, S, E, n, n, K, rho, nhi, nlo, OZK_ORDER_2SUM, G, ldg,
-                         nullptr, 0, ws, ws_bytes, st, Ssum, Ssum, true, pub);
+                         nullptr, 0, ws, ws_bytes, st, Ssum, Ssum, true, pub, dyn_zeroed);
 }
 
 int launch_gemm(const void* As, const int32_t* Ae, const void* Bs,
                 const int32_t* Be, int64_t N, int64_t M, int64_t K, int pipe,
                 int nhi, int nlo, int order, double* C, int64_t ldc,
                 void* ws, size_t ws_bytes, hipStream_t st, bool i8, int rho,
-                const int32_t* Asum, const int32_t* Bsum, FlagPub pub) {
+                const int32_t* Asum, const int32_t* Bsum, FlagPub pub, bool dyn_zeroed) {
   if (allpairs_schedule(pipe, nhi, nlo) && allpairs_order(pipe, nhi, nlo, order))
     return launch_allpairs(i8, pipe, As, Ae, Bs, Be, N, M, K, rho, nhi, nlo, order,
-                           C, ldc, nullptr, 0, ws, ws_bytes, st, Asum, Bsum, false, pub);
+                           C, ldc, nullptr, 0, ws, ws_bytes, st, Asum, Bsum, false, pub,
+                           dyn_zeroed);
   if (i8) {
     set_error("int8 slice planes need an all-pairs on-device schedule");
     return OZK_ERR_UNSUPPORTED;
