@@ -52,6 +52,10 @@ int extract(const double* X, int64_t rows, int64_t cols, int64_t ldx,
             int by_cols, int rho, int n0, int n1, void* S, int32_t* E,
             uint32_t* flags, void* ws, size_t wsb, hipStream_t st, bool i8,
             int32_t* sums, ZeroJobs zero = {}, bool zeroed = false);
+bool extract_pair_f32(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t N,
+                      int64_t K, int64_t M, int rho, int n0, int n1, void* SA, int32_t* EA,
+                      void* SB, int32_t* EB, uint32_t* flags, const ZeroJobs& zero,
+                      hipStream_t st);
 bool column_zero_jobs(int64_t arows, int64_t acols, int64_t rows, int64_t cols, int n0, int n1,
                       void* ws, int32_t* Sg, ZeroJobs& z);
 size_t extract_workspace_bytes(int64_t rows, int64_t cols, int by_cols, bool f64);
@@ -546,13 +550,18 @@ static int matmul_call(const double* A, int64_t lda, const double* B, int64_t ld
   zero.add((char*)gws + dyn_off, dyn_bytes);
   if (pipeline == OZK_PIPE_ONDEVICE) {
     rho = rho_generic(K, 24);
-    const bool zeroed = column_zero_jobs(N, K, K, M, n_hi, n_lo, tws, sb.sum, zero);
-    if ((rc = extract<float>(A, N, K, lda, 0, rho, n_hi, n_lo, sa.s, sa.e, flags,
-                             tws, tbytes, st, i8, sa.sum, zero)))
-      return rc;
-    if ((rc = extract<float>(B, K, M, ldb, 1, rho, n_hi, n_lo, sb.s, sb.e, flags,
-                             tws, tbytes, st, i8, sb.sum, {}, zeroed)))
-      return rc;
+    if (!i8 && extract_pair_f32(A, lda, B, ldb, N, K, M, rho, n_hi, n_lo, sa.s, sa.e, sb.s,
+                                sb.e, flags, zero, st)) {
+      OZK_LAUNCH_CHECK();
+    } else {
+      const bool zeroed = column_zero_jobs(N, K, K, M, n_hi, n_lo, tws, sb.sum, zero);
+      if ((rc = extract<float>(A, N, K, lda, 0, rho, n_hi, n_lo, sa.s, sa.e, flags,
+                               tws, tbytes, st, i8, sa.sum, zero)))
+        return rc;
+      if ((rc = extract<float>(B, K, M, ldb, 1, rho, n_hi, n_lo, sb.s, sb.e, flags,
+                               tws, tbytes, st, i8, sb.sum, {}, zeroed)))
+        return rc;
+    }
   } else {
     rho = rho_generic(K, 53);
     if ((rc = extract<double>(A, N, K, lda, 0, rho, n_hi, 0, sa.s, sa.e, flags,

@@ -196,15 +196,11 @@ __device__ __forceinline__ float fast_carry(float q, float k) {
 }
 
 template <typename W, int BLOCK, int EPT, int LPB, int FMT, int VEC>
-__global__ __launch_bounds__(BLOCK * LPB) void extract_lines_reg(
+__device__ __forceinline__ void lines_reg(
     const double* __restrict__ X, int64_t lines, int64_t len, int64_t ldx,
     int vec_ok, int rho, int n0, int n1, typename PlaneElem<FMT>::type* __restrict__ S,
     int64_t ld, int64_t plane, int32_t* __restrict__ E, int64_t eplane,
-    uint32_t* __restrict__ flags, int32_t* __restrict__ Sg, int ngroups, ZeroJobs zero) {
-  if ((int)blockIdx.x >= ngroups) {  // behind the lines' workgroups
-    run_zero_jobs(zero, (int)blockIdx.x - ngroups, (int)gridDim.x - ngroups);
-    return;
-  }
+    uint32_t* __restrict__ flags, int32_t* __restrict__ Sg, int64_t grp) {
   static_assert(VEC == 2 || VEC == 4, "VEC doubles are read as 16-byte pairs");
   const float qscale = ldexpf(1.0f, 24 - rho);
   constexpr int NP = Parts<W>::N;
@@ -217,7 +213,6 @@ __global__ __launch_bounds__(BLOCK * LPB) void extract_lines_reg(
     for (int i = threadIdx.x; i < kMaxPlanes * LPB; i += BLOCK * LPB) ssum[i] = 0;
   }
   const int t = threadIdx.x % BLOCK;
-  const int64_t grp = xcd_line(blockIdx.x, ngroups);
   const int64_t line = grp * LPB + threadIdx.x / BLOCK;
   const bool live = line < lines;
   // Plane offset of the thread's first element: BLOCK * VEC is a multiple of
@@ -369,6 +364,21 @@ __global__ __launch_bounds__(BLOCK * LPB) void extract_lines_reg(
       Sg[(i / LPB) * eplane + grp * LPB + i % LPB] =
           ssum[i] - i8_offset(rho) * (BLOCK * EPT * VEC);
   }
+}
+
+template <typename W, int BLOCK, int EPT, int LPB, int FMT, int VEC>
+__global__ __launch_bounds__(BLOCK * LPB) void extract_lines_reg(
+    const double* __restrict__ X, int64_t lines, int64_t len, int64_t ldx,
+    int vec_ok, int rho, int n0, int n1, typename PlaneElem<FMT>::type* __restrict__ S,
+    int64_t ld, int64_t plane, int32_t* __restrict__ E, int64_t eplane,
+    uint32_t* __restrict__ flags, int32_t* __restrict__ Sg, int ngroups, ZeroJobs zero) {
+  if ((int)blockIdx.x >= ngroups) {  // behind the lines' workgroups
+    run_zero_jobs(zero, (int)blockIdx.x - ngroups, (int)gridDim.x - ngroups);
+    return;
+  }
+  lines_reg<W, BLOCK, EPT, LPB, FMT, VEC>(X, lines, len, ldx, vec_ok, rho, n0, n1, S, ld,
+                                          plane, E, eplane, flags, Sg,
+                                          xcd_line(blockIdx.x, ngroups));
 }
 
 // Streaming extraction for lines too long for registers: every pass re-reads
@@ -909,15 +919,11 @@ constexpr int kPanelThreads = 512;
 constexpr int kPanelGroups = kPanelThreads / kPanelCols;  // 256 row groups
 
 template <int FMT, int RPT>
-__global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(4))) void extract_cols_panel(
+__device__ __forceinline__ void cols_panel(
     const double* __restrict__ X, int64_t K, int64_t M, int64_t ldx, int rho, int n0, int n1,
     typename PlaneElem<FMT>::type* __restrict__ S, int64_t ld, int64_t plane,
     int32_t* __restrict__ E, int64_t eplane, uint32_t* __restrict__ flags,
-    int32_t* __restrict__ Sg, int npanels, ZeroJobs zero) {
-  if ((int)blockIdx.x >= npanels) {  // behind the panels' workgroups
-    run_zero_jobs(zero, (int)blockIdx.x - npanels, (int)gridDim.x - npanels);
-    return;
-  }
+    int32_t* __restrict__ Sg, int64_t panel) {
   typedef typename PlaneElem<FMT>::type T;
   constexpr int NP = 2, NW = kPanelThreads / 64;
   constexpr int BYTES = RPT * (int)sizeof(T);  // plane bytes of a thread's rows
@@ -929,7 +935,6 @@ __global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(4
   if constexpr (FMT == kFmtI8) {
     for (int i = t; i < kMaxPlanes * kPanelCols; i += kPanelThreads) ssum[i] = 0;
   }
-  const int64_t panel = xcd_line(blockIdx.x, npanels);
   const int cl = t % kPanelCols;
   const int64_t line = panel * kPanelCols + cl;  // the thread's column
   const int64_t r0 = (int64_t)RPT * (t / kPanelCols);
@@ -1058,6 +1063,55 @@ __global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(4
     for (int i = t; i < (n0 + n1) * kPanelCols; i += kPanelThreads)
       Sg[(i / kPanelCols) * eplane + panel * kPanelCols + i % kPanelCols] =
           ssum[i] - i8_offset(rho) * (kPanelGroups * RPT);
+  }
+}
+
+template <int FMT, int RPT>
+__global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(4))) void extract_cols_panel(
+    const double* __restrict__ X, int64_t K, int64_t M, int64_t ldx, int rho, int n0, int n1,
+    typename PlaneElem<FMT>::type* __restrict__ S, int64_t ld, int64_t plane,
+    int32_t* __restrict__ E, int64_t eplane, uint32_t* __restrict__ flags,
+    int32_t* __restrict__ Sg, int npanels, ZeroJobs zero) {
+  if ((int)blockIdx.x >= npanels) {  // behind the panels' workgroups
+    run_zero_jobs(zero, (int)blockIdx.x - npanels, (int)gridDim.x - npanels);
+    return;
+  }
+  cols_panel<FMT, RPT>(X, K, M, ldx, rho, n0, n1, S, ld, plane, E, eplane, flags, Sg,
+                       xcd_line(blockIdx.x, npanels));
+}
+
+// One operand of extract_pair.
+struct PairOperand {
+  const double* X;
+  int64_t lines, ldx;
+  uint16_t* S;
+  int64_t plane;
+  int32_t* E;
+  int64_t eplane;
+  int groups;  // workgroups
+  int vec_ok;  // rows: 16-byte loads
+};
+
+// A's rows and B's columns (both of up to 4096 elements, BF16 planes) in one
+// launch: B's panels first (the longer ones), then A's lines, then the zero
+// jobs.  Small products are bound by the launches on their chain, and two
+// short kernels one after the other leave most of the chip idle twice: a high
+// product of 256^3 takes 29.0 us (34.8 with two launches), 1000 x 1531 x 777
+// 67.5 (74.8), and 4096^3 still gains 1% from the filled tails.
+template <int BLOCK, int EPT, int RPT>
+__global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(4))) void extract_pair(
+    PairOperand a, PairOperand b, int64_t len, int64_t ld, int rho, int n0, int n1,
+    uint32_t* __restrict__ flags, ZeroJobs zero) {
+  const int bid = (int)blockIdx.x;
+  if (bid < b.groups) {
+    cols_panel<kFmtBf16, RPT>(b.X, len, b.lines, b.ldx, rho, n0, n1, b.S, ld, b.plane, b.E,
+                              b.eplane, flags, nullptr, xcd_line(bid, b.groups));
+  } else if (bid < b.groups + a.groups) {
+    lines_reg<float, BLOCK, EPT, kPanelThreads / BLOCK, kFmtBf16, 2>(
+        a.X, a.lines, len, a.ldx, a.vec_ok, rho, n0, n1, a.S, ld, a.plane, a.E, a.eplane,
+        flags, nullptr, xcd_line(bid - b.groups, a.groups));
+  } else {
+    run_zero_jobs(zero, bid - b.groups - a.groups, (int)gridDim.x - b.groups - a.groups);
   }
 }
 
@@ -1501,6 +1555,46 @@ size_t extract_workspace_bytes(int64_t rows, int64_t cols, int by_cols, bool f64
   if (!f64 && gang_columns(rows)) return gang_workspace_bytes(rows, cols, kMaxSlices);
   return transpose_bytes(rows, cols) +
          (!f64 && gang_rows(rows) ? row_gang_bytes(cols, rows, kMaxSlices) : 0);
+}
+
+// FP32 extraction of A's rows (N x K) and B's columns (K x M) to BF16 planes
+// in one launch where both are at most kPairMax elements long; false (nothing
+// launched) otherwise.
+constexpr int64_t kPairMax = 4096;
+bool extract_pair_f32(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t N,
+                      int64_t K, int64_t M, int rho, int n0, int n1, void* SA, int32_t* EA,
+                      void* SB, int32_t* EB, uint32_t* flags, const ZeroJobs& zero,
+                      hipStream_t st) {
+  const int64_t ld = round_up(K, kKPad);
+  if (ld > kPairMax || !panel_columns(K)) return false;
+  auto operand = [&](const double* X, int64_t lines, int64_t ldx, void* S, int32_t* E, int per) {
+    PairOperand o;
+    o.X = X;
+    o.lines = lines;
+    o.ldx = ldx;
+    o.S = (uint16_t*)S;
+    o.eplane = round_up(lines, kLinePad);
+    o.plane = o.eplane * ld;
+    o.E = E;
+    o.groups = (int)(o.eplane / per);
+    o.vec_ok = (uintptr_t)X % 16 == 0 && ldx % 2 == 0 && K % 2 == 0;
+    return o;
+  };
+#define OZK_PAIR(BLOCK, EPT, RPT)                                                          \
+  do {                                                                                     \
+    const PairOperand a = operand(A, N, lda, SA, EA, kPanelThreads / BLOCK);               \
+    const PairOperand b = operand(B, M, ldb, SB, EB, kPanelCols);                          \
+    hipLaunchKernelGGL((extract_pair<BLOCK, EPT, RPT>),                                    \
+                       dim3((unsigned)(a.groups + b.groups + zero.groups(kPanelThreads))), \
+                       dim3(kPanelThreads), 0, st, a, b, K, ld, rho, n0, n1, flags, zero); \
+  } while (0)
+  // the shapes of launch_lines and launch_cols_panel
+  if (ld <= 256) OZK_PAIR(64, 2, 4);
+  else if (ld <= 1024) OZK_PAIR(128, 4, 4);
+  else if (ld <= 2048) OZK_PAIR(128, 8, 8);
+  else OZK_PAIR(256, 8, 16);
+#undef OZK_PAIR
+  return true;
 }
 
 // What a column gang extraction needs at zero.
