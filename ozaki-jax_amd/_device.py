@@ -45,25 +45,25 @@ _NO_GPU = ("ozaki_jax_amd needs a ROCm GPU; there is no CPU implementation "
 
 def _numpy_to_torch(a, dev):
     """A contiguous NumPy array as a device tensor.  Large ones go through
-    the pinned staging buffers (_hip), after torch's current stream has
-    drained (the copy runs on the null stream)."""
-    if a.nbytes < _hip._STAGE_MIN:
+    the pinned ring (_hip) on torch's current stream."""
+    if a.nbytes < _hip._COPY_MIN:
         return torch.from_numpy(a).to(dev)
     t = torch.empty(a.shape, dtype=_TORCH_DTYPES[a.dtype], device=dev)
-    torch.cuda.current_stream(dev).synchronize()
-    _hip._stager().to_device(t.data_ptr(), a)
+    with torch.cuda.device(dev):
+        _hip._stager().to_device(t.data_ptr(), a, torch.cuda.current_stream(dev).cuda_stream)
     return t
 
 
 def _torch_to_numpy(t):
     """A device tensor as a new NumPy array, large contiguous ones through the
-    pinned staging buffers."""
+    pinned ring (_hip) on torch's current stream."""
     if (not t.is_cuda or not t.is_contiguous() or t.dtype not in _NUMPY_DTYPES
-            or t.numel() * t.element_size() < _hip._STAGE_MIN):
+            or t.numel() * t.element_size() < _hip._COPY_MIN):
         return t.cpu().numpy()
     out = np.empty(tuple(t.shape), _NUMPY_DTYPES[t.dtype])
-    torch.cuda.current_stream(t.device).synchronize()
-    _hip._stager().to_host(out, t.data_ptr())
+    with torch.cuda.device(t.device):
+        _hip._stager().to_host(out, t.data_ptr(),
+                               torch.cuda.current_stream(t.device).cuda_stream)
     return out
 
 

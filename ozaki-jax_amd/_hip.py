@@ -11,17 +11,16 @@ Device memory comes from a caching pool: blocks are rounded to size classes
 and kept for reuse after their arrays are garbage collected, so repeated
 calls of one shape allocate nothing after the first.
 
-Host copies of large arrays go through two pinned staging buffers: host
-threads copy one chunk between the NumPy array and a staging buffer while
-the DMA engine moves the other (a direct copy from pageable memory, and
-the page faults of a fresh output array, are otherwise serial).
+Host copies of 1 MiB and more go through pinned memory: the
+library's host threads move bytes between the NumPy array and it while
+others are on the link (a direct copy from pageable memory,
+and the page faults of a fresh output array, are otherwise serial).
 """
 
 import atexit
 import ctypes
 import os
 import threading
-from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 
@@ -141,70 +140,95 @@ class _Runtime:
         self.check(self.h.hipEventDestroy(e), "hipEventDestroy")
 
 
-# Host copies of at least _STAGE_MIN bytes are staged in _STAGE_CHUNK pieces.
+# Host copies of at least _COPY_MIN bytes go through pinned memory
+# (_Stager); smaller ones are as fast as the runtime's own copies.  Those above
+# _SLOTS * _SLOT bytes take the larger slots.  Products whose halves reach _STAGE_MIN bytes
+# run in two halves (matmul).
+_COPY_MIN = 1 << 20
+_SLOTS, _SLOT = 8, 4 << 20
+_BIG_SLOTS, _BIG_SLOT = 4, 32 << 20
 _STAGE_MIN = 32 << 20
 _STAGE_CHUNK = 64 << 20
 
 
-class _Stager:
-    """Two pinned buffers of `chunk` bytes (allocated once, kept for the
-    process), an event per buffer on the null stream, and a thread pool for
-    the host-side copies.  One transfer at a time (a lock)."""
+class _Slots:
+    """Pinned slots with an event each (ozk_copy_slots).  One transfer at a
+    time (a lock)."""
 
-    def __init__(self, rt, chunk=_STAGE_CHUNK):
-        self.rt, self.chunk = rt, int(chunk)
-        self.buf = [rt.host_malloc(self.chunk) for _ in range(2)]
-        self.ev = [rt.event() for _ in range(2)]
-        self.nthreads = max(1, min(8, os.cpu_count() or 1))
-        self.pool = ThreadPoolExecutor(self.nthreads)
+    def __init__(self, rt, slot, slots):
+        self.slot, self.slots, self.first = int(slot), int(slots), 0
+        self.buf = rt.host_malloc(self.slot * self.slots)
+        self.ev = (ctypes.c_void_p * self.slots)(*[rt.event() for _ in range(self.slots)])
         self.lock = threading.Lock()
 
-    def _host_copy(self, dst, src):
-        """dst[:] = src for two flat uint8 arrays, split over the threads."""
-        n = dst.size
-        step = -(-n // self.nthreads)
-        parts = [(a, min(a + step, n)) for a in range(0, n, step)]
-        list(self.pool.map(lambda ab: np.copyto(dst[ab[0]:ab[1]], src[ab[0]:ab[1]]), parts))
-
-    def _staging(self, i, n):
-        return np.ctypeslib.as_array((ctypes.c_uint8 * n).from_address(self.buf[i]))
-
-    def to_device(self, dev_ptr, host):
-        """host: a C-contiguous array; its bytes to dev_ptr."""
-        src = host.reshape(-1).view(np.uint8)
+    def copy(self, down, dev_ptr, host, threads, stream):
         with self.lock:
-            try:
-                for k, a in enumerate(range(0, src.size, self.chunk)):
-                    b = min(a + self.chunk, src.size)
-                    i = k & 1
-                    if k >= 2:
-                        self.rt.wait(self.ev[i])  # the DMA of chunk k - 2 has read buffer i
-                    self._host_copy(self._staging(i, b - a), src[a:b])
-                    self.rt.copy_async(dev_ptr + a, self.buf[i], b - a, _H2D)
-                    self.rt.record(self.ev[i])
-            finally:  # no copy may still read the buffers once the lock is free
-                self.rt.sync()
+            first = self.first
+            self.first = (first + -(-host.nbytes // self.slot)) % self.slots
+            _lib.check(_lib.load().ozk_copy_slots(
+                down, dev_ptr, host.ctypes.data, host.nbytes, self.buf, self.slot, self.slots,
+                first, self.ev, threads, stream))
 
-    def to_host(self, out, dev_ptr):
-        """out: a C-contiguous array; its bytes from dev_ptr."""
-        dst = out.reshape(-1).view(np.uint8)
+    def release(self, h):
+        h.hipHostFree(self.buf)
+        for e in self.ev:
+            h.hipEventDestroy(e)
+
+
+class _Stager:
+    """Pinned memory of the library's staged copies, allocated once per device
+    and kept for the process: slots for the way up, as much memory with a
+    flag word and a device counter per 512 KiB for the way down
+    (ozk_copy_to_host), and larger slots for large transfers either way.  One
+    transfer at a time in each (a lock)."""
+
+    def __init__(self, rt, slot=_SLOT, slots=_SLOTS):
+        self.rt, self.size = rt, int(slot) * int(slots)
+        self.up, self.big = _Slots(rt, slot, slots), None
+        self.down = rt.host_malloc(self.size)
+        words = 4 * (self.size >> 19)
+        self.flags, self.counts = rt.host_malloc(words), rt.malloc(words)
+        rt.memset(self.counts, 0, words)
+        rt.sync()
+        ctypes.memset(self.flags, 0, words)
+        for p in (self.up.buf, self.down):  # map the pages now, not call by call
+            ctypes.memset(p, 0, self.size)
+        self.max_threads = max(1, min(8, os.cpu_count() or 1))
+        self.lock = threading.Lock()
+
+    def _threads(self, nbytes):
+        return min(self.max_threads, 1 + (nbytes >> 20))
+
+    def _big(self):
         with self.lock:
-            chunks = [(a, min(a + self.chunk, dst.size)) for a in range(0, dst.size, self.chunk)]
-            try:
-                for k, (a, b) in enumerate(chunks[:2]):
-                    self.rt.copy_async(self.buf[k], dev_ptr + a, b - a, _D2H)
-                    self.rt.record(self.ev[k])
-                for k, (a, b) in enumerate(chunks):
-                    i = k & 1
-                    self.rt.wait(self.ev[i])
-                    self._host_copy(dst[a:b], self._staging(i, b - a))
-                    if k + 2 < len(chunks):  # buffer i is free again
-                        a2, b2 = chunks[k + 2]
-                        self.rt.copy_async(self.buf[i], dev_ptr + a2, b2 - a2, _D2H)
-                        self.rt.record(self.ev[i])
-            except BaseException:
-                self.rt.sync()  # no copy may still write the buffers once the lock is free
-                raise
+            if self.big is None:
+                self.big = _Slots(self.rt, _BIG_SLOT, _BIG_SLOTS)
+            return self.big
+
+    def to_device(self, dev_ptr, host, stream=None):
+        """host: a C-contiguous array, whose bytes go to dev_ptr on `stream`.
+        They have been read when this returns; the copy may still run."""
+        slots = self.up if host.nbytes <= _SLOT * _SLOTS else self._big()
+        slots.copy(0, dev_ptr, host, self._threads(host.nbytes), stream)
+
+    def to_host(self, out, dev_ptr, stream=None):
+        """out: a C-contiguous array, filled from dev_ptr behind the work
+        queued on `stream`."""
+        if out.nbytes > _SLOT * _SLOTS:
+            self._big().copy(1, dev_ptr, out, self._threads(out.nbytes), stream)
+            return
+        with self.lock:
+            _lib.check(_lib.load().ozk_copy_to_host(
+                out.ctypes.data, dev_ptr, out.nbytes, self.down, self.size, self.flags,
+                self.counts, self._threads(out.nbytes), stream))
+
+    def release(self, h):
+        self.up.release(h)
+        if self.big is not None:
+            self.big.release(h)
+        for p in (self.down, self.flags):
+            h.hipHostFree(p)
+        h.hipFree(self.counts)
 
 
 class _Pool:
@@ -310,7 +334,7 @@ class DeviceArray:
         a = np.ascontiguousarray(a)
         d = cls(a.shape, a.dtype)
         assert d.nbytes == a.nbytes
-        if a.nbytes >= _STAGE_MIN:
+        if a.nbytes >= _COPY_MIN:
             _stager().to_device(d.data_ptr(), a)
         else:
             _rt().copy(d.data_ptr(), a.ctypes.data, a.nbytes, _H2D)
@@ -325,7 +349,7 @@ class DeviceArray:
             full = np.empty((self.shape[0], self.ld), self.dtype)
             _rt().copy(full.ctypes.data, self.data_ptr(), self.nbytes, _D2H)
             out[:] = full[:, :self.shape[1]]
-        elif out.nbytes >= _STAGE_MIN:
+        elif out.nbytes >= _COPY_MIN:
             _stager().to_host(out, self.data_ptr())
         else:
             _rt().copy(out.ctypes.data, self.data_ptr(), out.nbytes, _D2H)
@@ -449,21 +473,18 @@ def _release_at_exit():
     unusable by then."""
     with _state_lock:
         st = dict(_state)
-        for k in ("stager", "blas", "cstream"):
-            _state.pop(k, None)
+        for k in st:
+            if k not in ("rt", "pool"):
+                _state.pop(k, None)
     rt = st.get("rt")
     if rt is None:
         return
     h = rt.h
     try:
         h.hipDeviceSynchronize()
-        stager = st.get("stager")
-        if stager is not None:
-            stager.pool.shutdown(wait=True)
-            for b in stager.buf:
-                h.hipHostFree(b)
-            for e in stager.ev:
-                h.hipEventDestroy(e)
+        for stager in st.values():
+            if isinstance(stager, _Stager):
+                stager.release(h)
         blas_ = st.get("blas")
         if blas_ is not None:
             blas_.b.rocblas_destroy_handle(blas_.h)
@@ -491,7 +512,8 @@ def _pool():
 
 
 def _stager():
-    return _get("stager", lambda: _Stager(_rt()))
+    """The current device's ring."""
+    return _get(("stager", _rt().device()), lambda: _Stager(_rt()))
 
 
 def compute_stream():

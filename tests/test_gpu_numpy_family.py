@@ -153,6 +153,29 @@ def test_staged_transfers_round_trip(no_torch, nbytes, chunk):
     assert np.array_equal(out, a), "D2H"
 
 
+@pytest.mark.parametrize("nbytes", [8, 1 << 19, (1 << 19) + 8, 3 << 19, (10 << 19) - 8])
+def test_staged_transfers_wrap_a_small_ring(no_torch, nbytes):
+    """Four half-MiB slots (two pieces a batch down): copies of up to ten
+    pieces, one after the other without a wait between them, from and to
+    arrays of their own, 16-byte aligned or not."""
+    from ozaki_jax_amd import _hip
+    st = _hip._Stager(_hip._rt(), 1 << 19, 4)
+    rng = np.random.RandomState(nbytes % 1000)
+    arrays = [rng.randint(0, 1 << 60, nbytes // 8) for _ in range(3)]
+    case(f"staged copies of {nbytes} bytes through four slots")
+    devs = [_hip.DeviceArray(a.shape, a.dtype) for a in arrays]
+    for a, d in zip(arrays, devs):
+        st.to_device(d.data_ptr(), a)
+    for a, d in zip(arrays, devs):
+        out = np.full_like(a, -1)
+        st.to_host(out, d.data_ptr())
+        assert np.array_equal(out, a)
+        for shift in (8, 3):
+            out = np.full(a.nbytes - shift, 255, np.uint8)
+            st.to_host(out, d.data_ptr() + shift)
+            assert np.array_equal(out, a.view(np.uint8)[shift:])
+
+
 def test_large_array_round_trip(no_torch):
     """An array above the staging threshold goes through the default stager
     both ways."""
