@@ -264,7 +264,8 @@ constexpr int ap_rb(int nhi, int nlo, int b0, int b1, bool sym) {
 // (kFirst: no fold state to load) and ends it (kLast: C is written, not the
 // state), how many blocks the schedule folds (kNBlk) and, for the 2Sum
 // state, the blocks folded before and after it (kDone0, kDone1).
-template <int PIPE, int NHI, int NLO, int B0, int B1, bool SYM = false>
+// SMALL: tiles of 32 rows (RB = 1), for products of few tiles (small_form).
+template <int PIPE, int NHI, int NLO, int B0, int B1, bool SYM = false, bool SMALL = false>
 struct Sweep {
   static_assert(PIPE == OZK_PIPE_ONDEVICE, "sweeps cover the on-device schedule");
   static constexpr bool kRect = false, kFirst = B0 == 0, kLast = B1 == 2;
@@ -280,7 +281,7 @@ struct Sweep {
                                                : NHI * NHI + 2 * NHI * NLO);
   static constexpr int NP = P1 - P0;  // pairs of the sweep
   static constexpr int S = NA + NB;   // LDS slots per stage
-  static constexpr int RB = ap_rb(NHI, NLO, B0, B1, SYM);  // row blocks per wave
+  static constexpr int RB = SMALL ? 1 : ap_rb(NHI, NLO, B0, B1, SYM);  // row blocks per wave
   static constexpr int TM = 32 * RB;                     // tile rows
   static constexpr int FA = 2 * RB;                      // fragments per A slot
   static constexpr int NFRAG = NA * FA + NB * 4;         // fragments per stage
@@ -300,8 +301,8 @@ struct Sweep {
 // of the first group's pairs.  The FP64 orders fold the products of a group
 // into one running sum, so the sweeps, which cut between groups, carry that
 // sum alone.
-template <int N, int G0, int G1>
-struct Sweep<OZK_PIPE_HOST, N, 0, G0, G1, false> {
+template <int N, int G0, int G1, bool SMALL>
+struct Sweep<OZK_PIPE_HOST, N, 0, G0, G1, false, SMALL> {
   static constexpr bool kRect = false, kFirst = G0 == 0, kLast = G1 == N - 1;
   static constexpr bool kMid0 = false, kMid1 = false;
   static constexpr int kNBlk = 1, kDone0 = 0, kDone1 = 0;
@@ -310,7 +311,7 @@ struct Sweep<OZK_PIPE_HOST, N, 0, G0, G1, false> {
   static constexpr int P1 = (G1 + 1) * N - G1 * (G1 + 1) / 2;
   static constexpr int NP = P1 - P0;
   static constexpr int S = NA + NB;
-  static constexpr int RB = ap_rb_of(NP, NA, NB, false);
+  static constexpr int RB = SMALL ? 1 : ap_rb_of(NP, NA, NB, false);
   static constexpr int TM = 32 * RB;
   static constexpr int FA = 2 * RB;
   static constexpr int NFRAG = NA * FA + NB * 4;
@@ -354,7 +355,7 @@ constexpr int kRfDone0 = 7;         // bits 7-8: blocks folded before it
 constexpr int kRfDone1 = 9;         // bits 9-10: ... and after it
 
 template <int NA_, int NB_>
-struct Sweep<kPipeRect, NA_, NB_, 0, 0, false> {
+struct Sweep<kPipeRect, NA_, NB_, 0, 0, false, false> {
   static constexpr bool kRect = true, kFirst = false, kLast = false;
   static constexpr bool kMid0 = false, kMid1 = false;
   static constexpr int kNBlk = 3, kDone0 = 0, kDone1 = 0;
@@ -505,7 +506,7 @@ __device__ __forceinline__ void stage_dma(const char* At, int64_t aplane,
 #pragma unroll
     for (int gg = 0; gg < (FA + 3) / 4; ++gg) {
       const int g = wave + 4 * gg;
-      if (gg == 0 || g < FA) {  // uniform
+      if ((gg == 0 && FA >= 4) || g < FA) {  // uniform
         const int gs = g < agroups ? g : agroups - 1;
         dma16(__builtin_amdgcn_readfirstlane(buf_lds + (FA * slot + g) * 1024),
               (const void*)(At + slot * aplane + qa + (int64_t)gs * 1024), lane_bytes);
@@ -518,11 +519,12 @@ __device__ __forceinline__ void stage_dma(const char* At, int64_t aplane,
           (const void*)(Bt + slot * bplane + qb), lane_bytes);
 }
 
-// Loads a DMA wave issues per stage: one per B slot and one or two per A
-// slot (waves 0 .. FA - 5 take two A groups).
+// Loads a DMA wave issues per stage: one per B slot and up to two per A
+// slot (FA = 6: waves 0 and 1 take two A groups; FA = 2: they take one and
+// waves 2 and 3 none).
 template <int NA, int NB, int FA>
 __host__ __device__ constexpr int stage_loads(int wave) {
-  return NB + NA * (wave + 4 < FA ? 2 : 1);
+  return NB + NA * ((wave < FA ? 1 : 0) + (wave + 4 < FA ? 1 : 0));
 }
 
 // vmcnt wait before consuming a stage: the loads of the `later` stages
@@ -773,7 +775,7 @@ __device__ __forceinline__ void tile_epilogue(
 // sequence through the LDS ring, so the loads of a tile's first stages are
 // issued during the previous tile's last stages and epilogue.
 
-template <class Op, int PIPE, int NHI, int NLO, int ORDER, int B0, int B1, bool SYM>
+template <class Op, int PIPE, int NHI, int NLO, int ORDER, int B0, int B1, bool SYM, bool SMALL>
 __global__ __launch_bounds__(kThreads16) void gemm_allpairs(
     const char* __restrict__ As, const int32_t* __restrict__ Ae,
     const char* __restrict__ Bs, const int32_t* __restrict__ Be,
@@ -781,7 +783,7 @@ __global__ __launch_bounds__(kThreads16) void gemm_allpairs(
     float unit2, double* __restrict__ C, int64_t ldc, float* __restrict__ P,
     int64_t ldp, char* __restrict__ state, int tail_P, uint32_t* __restrict__ part,
     I8Fix fix, uint32_t* __restrict__ dyn, int dyn_nstat, int rflags, FlagPub pub) {
-  typedef Sweep<PIPE, NHI, NLO, B0, B1, SYM> SW;
+  typedef Sweep<PIPE, NHI, NLO, B0, B1, SYM, SMALL> SW;
   constexpr int NA = SW::NA, NB = SW::NB, NP = SW::NP, RB = SW::RB, FA = SW::FA;
   constexpr int kBuf = SW::NFRAG * 64;  // uint4 per stage buffer
   static_assert(kRing == 4, "wait_stage assumes 4 stage buffers");
@@ -963,7 +965,7 @@ __global__ __launch_bounds__(kThreads16) void gemm_allpairs(
   for (int64_t g = 0; g < total; ++g) {
     const int64_t later = total - 1 - g < kRing - 2 ? total - 1 - g : kRing - 2;
     if (dma_wave) {
-      if (wave + 4 < FA) wait_stage<stage_loads<NA, NB, FA>(0)>(later);
+      if (FA % 4 != 0 && wave < 2) wait_stage<stage_loads<NA, NB, FA>(0)>(later);
       else wait_stage<stage_loads<NA, NB, FA>(3)>(later);
     }
     __syncthreads();
@@ -1000,13 +1002,13 @@ __global__ __launch_bounds__(kThreads16) void gemm_allpairs(
 // adds up a sixth-or-so of the lane's 2 NP accumulator vectors over all
 // pieces (several pieces' loads in flight), leaves the sums in LDS, and
 // wave 0 folds them.  Tail tile t is tile tile0 + t of the all-pairs order.
-template <class Op, int PIPE, int NHI, int NLO, int ORDER, int B0, int B1, bool SYM>
+template <class Op, int PIPE, int NHI, int NLO, int ORDER, int B0, int B1, bool SYM, bool SMALL>
 __global__ __launch_bounds__(kThreads16) void gemm_tail_fixup(
     const uint32_t* __restrict__ part, int tail_P, int tile0,
     const int32_t* __restrict__ Ae, const int32_t* __restrict__ Be, int64_t N,
     int64_t M, int64_t a_lines, int64_t b_lines, float unit2, double* __restrict__ C,
     int64_t ldc, float* __restrict__ P, int64_t ldp, char* __restrict__ state, I8Fix fix) {
-  typedef Sweep<PIPE, NHI, NLO, B0, B1, SYM> SW;
+  typedef Sweep<PIPE, NHI, NLO, B0, B1, SYM, SMALL> SW;
   typedef typename Op::acc_t V;
   constexpr int NP = SW::NP, RB = SW::RB, NV = RB * NP;  // accumulator vectors per lane
   constexpr int PER = (NV + 7) / 8;                      // vectors per wave
@@ -1214,6 +1216,22 @@ constexpr bool allpairs_preset(int nhi, int nlo) {
 }
 
 
+// Schedules and orders with kernels of 32-row tiles: the presets in the
+// on-device orders, the host schedules of 8 and 9 slices (those its slice
+// budget asks for).  They serve products whose usual tiles would leave half
+// of the CUs or more idle (use_small): a stage of such a tile has half the
+// MFMAs and its fold half the elements, so it ends sooner on twice the CUs.
+// Whole calls, 64-row tiles -> these, without a split of K (us): 24 pairs
+// 256 x 4096 x 256 133 -> 97, 64 x 64 x 64 29.5 -> 30; 65 pairs 512^3 79 -> 63;
+// host schedule of 8 slices 256^3 117 -> 109.
+constexpr int kSmallTM = 32;
+constexpr bool small_form(int pipe, int nhi, int nlo, int order) {
+  return pipe == OZK_PIPE_HOST
+             ? (nhi == 8 || nhi == 9) && (order == OZK_ORDER_HOST_JAX || order == OZK_ORDER_HOST_NP)
+             : pipe == OZK_PIPE_ONDEVICE && allpairs_preset(nhi, nlo) &&
+                   (order == OZK_ORDER_2SUM || order == OZK_ORDER_BLOCK64);
+}
+
 // Dynamic tail (gemm_allpairs): with R = ntiles / cus whole rounds, the
 // last ceil(R / kDynDiv) of them are handed out at run time from one counter
 // per XCD and sweep (kDynBytes, zeroed before the launch).  Needs at least
@@ -1256,6 +1274,7 @@ struct ApArgs {
   char* state;
   I8Fix fix;
   FlagPub pub;  // taken by the schedule's first sweep
+  bool small;   // kSmallTM-row tiles
 };
 
 // One sweep's kernel on operands As .. fix (the rectangle sweeps pass them
@@ -1265,11 +1284,12 @@ struct ApArgs {
 // along K instead, on the grid the plan of launch_allpairs chose, and then
 // runs the fixup.  (Sweeps of multi-sweep schedules do not split: there the
 // fixups cost about what the split saves.)
-template <class Op, int PIPE, int NHI, int NLO, int ORDER, int B0, int B1, bool SYM>
+template <class Op, int PIPE, int NHI, int NLO, int ORDER, int B0, int B1, bool SYM,
+          bool SMALL = false>
 static void launch_sweep_kernel(const ApArgs& a, const char* As, const int32_t* Ae,
                                 const char* Bs, const int32_t* Be, const I8Fix& fix,
                                 int ordinal, int rflags) {
-  typedef Sweep<PIPE, NHI, NLO, B0, B1, SYM> SW;
+  typedef Sweep<PIPE, NHI, NLO, B0, B1, SYM, SMALL> SW;
   const int64_t nt = allpairs_ntiles(a.N, a.M, SYM, SW::TM);
   dim3 grid((unsigned)(nt < a.cus ? nt : a.cus));
   int tail_P = 0, tile0 = 0;
@@ -1290,13 +1310,13 @@ static void launch_sweep_kernel(const ApArgs& a, const char* As, const int32_t* 
     nstat = dyn_static_rounds(nt, (int)grid.x, a.nst);
     if (nstat > 0) dyn = a.dyn + kXcds * ordinal;
   }
-  hipLaunchKernelGGL((gemm_allpairs<Op, PIPE, NHI, NLO, ORDER, B0, B1, SYM>), grid,
+  hipLaunchKernelGGL((gemm_allpairs<Op, PIPE, NHI, NLO, ORDER, B0, B1, SYM, SMALL>), grid,
                      dim3(kThreads16), 0, a.st, As, Ae, Bs, Be, a.N, a.M, a.nst, a.al, a.bl,
                      a.unit2, a.C, a.ldc, a.P, a.ldp, a.state, tail_P, part, fix, dyn, nstat,
                      rflags, SW::kFirst || (rflags & kRfFirst) ? a.pub : FlagPub{});
   if constexpr (SW::kFirst && SW::kLast) {
     if (tail_P > 1)
-      hipLaunchKernelGGL((gemm_tail_fixup<Op, PIPE, NHI, NLO, ORDER, B0, B1, SYM>),
+      hipLaunchKernelGGL((gemm_tail_fixup<Op, PIPE, NHI, NLO, ORDER, B0, B1, SYM, SMALL>),
                          dim3((unsigned)(tail_T * 8)), dim3(kThreads16), 0, a.st, part, tail_P,
                          tile0, Ae, Be, a.N, a.M, a.al, a.bl, a.unit2, a.C, a.ldc, a.P, a.ldp,
                          a.state, fix);
@@ -1307,6 +1327,13 @@ static void launch_sweep_kernel(const ApArgs& a, const char* As, const int32_t* 
 // first block or group).
 template <class Op, int PIPE, int NHI, int NLO, int ORDER, int B0, int B1, bool SYM = false>
 static void launch_sweep_of(const ApArgs& a) {
+  if constexpr (!SYM && small_form(PIPE, NHI, NLO, ORDER)) {
+    if (a.small) {
+      launch_sweep_kernel<Op, PIPE, NHI, NLO, ORDER, B0, B1, SYM, true>(a, a.As, a.Ae, a.Bs,
+                                                                        a.Be, a.fix, B0, 0);
+      return;
+    }
+  }
   launch_sweep_kernel<Op, PIPE, NHI, NLO, ORDER, B0, B1, SYM>(a, a.As, a.Ae, a.Bs, a.Be, a.fix,
                                                               B0, 0);
 }
@@ -1594,10 +1621,24 @@ size_t gemm_state_bytes(int64_t N, int64_t M, int pipe, int nhi, int nlo, int or
 // K-split of the tail.  With R = ntiles / cus whole rounds of one tile per
 // workgroup and T = ntiles % cus tiles left, the last round would keep T
 // CUs busy while the others idle.  Instead each tail tile is split along K
-// into P = min(cus / T, nst / kMinPieceStages) pieces, one per workgroup,
-// whose raw sums gemm_tail_fixup adds up and folds.  Single-sweep schedules
-// only; needs T * P * NP * RB * 4 * kThreads16 * 4 bytes of workspace.
-constexpr int kMinPieceStages = 16;
+// into P <= cus / T pieces, one per workgroup, whose raw sums gemm_tail_fixup
+// adds up and folds.  Single-sweep schedules only; needs
+// T * P * NP * RB * 4 * kThreads16 * 4 bytes of workspace.
+//
+// P is the one that minimises nst / P + split_cost(), both in stages of one
+// tile: the sums written and read again (200 KB RB per piece for 24 pairs), the
+// fixup's launch and its walk over the P pieces of a tile.  The pairs of the
+// schedule do not enter, since the stage and the sums both grow with them.
+// Fitted to the whole call at 24 pairs (us; without a split / the P it picks / the
+// P = min(cus / T, nst / 16) of before):
+//   RB 1, nst 64:  T 2 55 / 36 / 38,  T 64 58 / 53 / 54,  T 128 60 / 60 / 68
+//   RB 1, nst 32:  T 32 37 / 37 / 43,  T 128 42 / 42 / 55
+//   RB 1, nst 128: T 8 98 / 47 / 47,  T 32 97 / 55 / 56,  T 128 102 / 91 / 91
+//   RB 2, nst 64:  T 16 152 / 137 / 137,  T 64 153 / 153 / 173
+//   RB 2, nst 128: T 16 281 / 222 / 224,  T 64 283 / 259 / 275
+static double split_cost(int64_t T, int64_t P, int rb) {
+  return (rb == 1 ? 1.0 : 1.6) * (12.0 + (double)P + (double)(T * P) / 10);
+}
 
 struct TailPlan {
   int P = 0;        // pieces per tail tile (0: no split)
@@ -1610,7 +1651,12 @@ static TailPlan plan_tail(int64_t ntiles, int cus, int64_t nst, int np, int rb) 
   TailPlan tp;
   const int64_t R = ntiles / cus, T = ntiles % cus;
   if (T == 0) return tp;
-  const int64_t P = cus / T < nst / kMinPieceStages ? cus / T : nst / kMinPieceStages;
+  int64_t P = 1;
+  double best = (double)nst;
+  for (int64_t p = 2; p <= cus / T && p <= nst; ++p) {
+    const double c = (double)nst / (double)p + split_cost(T, p, rb);
+    if (c < best) best = c, P = p;
+  }
   if (P < 2) return tp;
   tp.P = (int)P;
   tp.T = T;
@@ -1649,6 +1695,15 @@ static int allpairs_tm(int pipe, int nhi, int nlo, bool sym) {
                                      : ap_rb(nhi, nlo, 0, 2, sym));
 }
 
+// Whether an N x M product takes the 32-row tiles: if all of them fit the CUs
+// at once.  (A second round would cost more than the larger tiles: a stage
+// takes 0.6 us at 32 rows and 0.96 at 64 for 24 pairs, since a stage of 32 rows
+// is bound by LDS, 110 KB a stage, and no longer by its MFMAs.)
+static bool use_small(int64_t N, int64_t M, int pipe, int nhi, int nlo, int order, bool sym) {
+  return !sym && small_form(pipe, nhi, nlo, order) &&
+         allpairs_ntiles(N, M, false, kSmallTM) <= cu_count();
+}
+
 static int64_t allpairs_nst(int64_t K, bool i8) {
   // chunks per line: round_up(K, kKPad) elements of 1 or 2 bytes
   return round_up(K, kKPad) * (i8 ? 1 : 2) / kChunkBytes;
@@ -1659,7 +1714,9 @@ static int64_t allpairs_nst(int64_t K, bool i8) {
 size_t gemm_tail_bytes(int64_t N, int64_t M, int64_t K, int pipe, int nhi, int nlo,
                        bool sym, bool i8) {
   if (!allpairs_schedule(pipe, nhi, nlo) || allpairs_sweeps(pipe, nhi, nlo) != 1) return 0;
-  const int tm = allpairs_tm(pipe, nhi, nlo, sym);
+  const int tm = use_small(N, M, pipe, nhi, nlo, OZK_ORDER_2SUM, sym)
+                     ? kSmallTM
+                     : allpairs_tm(pipe, nhi, nlo, sym);
   return plan_tail(allpairs_ntiles(N, M, sym, tm), cu_count(), allpairs_nst(K, i8),
                    pair_count(pipe, nhi, nlo), tm / 32)
       .bytes;
@@ -1688,7 +1745,8 @@ static int launch_allpairs(bool i8, int pipe, const void* As, const int32_t* Ae,
   }
   ApArgs a;
   const int64_t al = round_up(N, kLinePad), bl = round_up(M, kLinePad);
-  const int tmr = allpairs_tm(pipe, nhi, nlo, sym);
+  a.small = use_small(N, M, pipe, nhi, nlo, order, sym);
+  const int tmr = a.small ? kSmallTM : allpairs_tm(pipe, nhi, nlo, sym);
   const int64_t ntiles = allpairs_ntiles(N, M, sym, tmr);
   OZK_CHECK_ARG(ntiles < (1ll << 31), "problem too large for one launch");
   // persistent: one workgroup per CU (the 160 KiB ring fills its LDS)
