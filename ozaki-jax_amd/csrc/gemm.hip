@@ -1629,15 +1629,18 @@ size_t gemm_state_bytes(int64_t N, int64_t M, int pipe, int nhi, int nlo, int or
 // tile: the sums written and read again (200 KB RB per piece for 24 pairs), the
 // fixup's launch and its walk over the P pieces of a tile.  The pairs of the
 // schedule do not enter, since the stage and the sums both grow with them.
-// Fitted to the whole call at 24 pairs (us; without a split / the P it picks / the
-// P = min(cus / T, nst / 16) of before):
-//   RB 1, nst 64:  T 2 55 / 36 / 38,  T 64 58 / 53 / 54,  T 128 60 / 60 / 68
-//   RB 1, nst 32:  T 32 37 / 37 / 43,  T 128 42 / 42 / 55
+// Pieces of kMinPieceStages or more keep the workspace no larger than that of
+// P = min(cus / T, nst / kMinPieceStages) on the usual tiles.
+// Fitted to the whole call at 24 pairs (us; without a split / the P it picks / that P):
+//   RB 1, nst 64:  T 2 55 / 38 / 38,  T 64 58 / 53 / 54,  T 128 60 / 60 / 68
+//   RB 1, nst 32:  T 2 33 / 33 / 34,  T 32 37 / 37 / 43,  T 128 42 / 42 / 55
 //   RB 1, nst 128: T 8 98 / 47 / 47,  T 32 97 / 55 / 56,  T 128 102 / 91 / 91
 //   RB 2, nst 64:  T 16 152 / 137 / 137,  T 64 153 / 153 / 173
 //   RB 2, nst 128: T 16 281 / 222 / 224,  T 64 283 / 259 / 275
+constexpr int kMinPieceStages = 16;
+
 static double split_cost(int64_t T, int64_t P, int rb) {
-  return (rb == 1 ? 1.0 : 1.6) * (12.0 + (double)P + (double)(T * P) / 10);
+  return (rb == 1 ? 1.0 : 1.6) * (15.0 + (double)P + (double)(T * P) / 10);
 }
 
 struct TailPlan {
@@ -1653,7 +1656,7 @@ static TailPlan plan_tail(int64_t ntiles, int cus, int64_t nst, int np, int rb) 
   if (T == 0) return tp;
   int64_t P = 1;
   double best = (double)nst;
-  for (int64_t p = 2; p <= cus / T && p <= nst; ++p) {
+  for (int64_t p = 2; p <= cus / T && p <= nst / kMinPieceStages; ++p) {
     const double c = (double)nst / (double)p + split_cost(T, p, rb);
     if (c < best) best = c, P = p;
   }

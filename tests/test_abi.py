@@ -122,6 +122,12 @@ def test_workspace_sizes(lib):
     assert ws >= 8 * 1000 * 64
 
 
+def test_matmul_split_fits_the_no_allocation_workspace(lib):
+    # at the edge of what ozk_matmul_noalloc accepts (128 MiB), with a split tail
+    for N, K, M, nh, nl in ((4724, 1540, 4574, 2, 2), (6678, 1628, 298, 4, 1)):
+        assert lib.ozk_matmul_workspace_bytes(N, K, M, 0, nh, nl) <= 128 << 20
+
+
 def test_residual_workspace_bytes(lib):
     # the fused row kernels need no workspace: high / medium up to K = 16384,
     # max up to 8192, up to 4 right-hand sides; other cases take the
