@@ -72,9 +72,9 @@ __device__ __forceinline__ uint32_t lu_wave_reduce(uint32_t u) {
 // Measured with the row slots a compile-time count, the loads and stores
 // four lanes a row and the permutation composed in parallel (us a panel,
 // unrolled -> rolled): 4096 rows 108 -> 88, 2048 71 -> 45, 512 46 -> 30; n =
-// 4096 factored in 9.1 ms (12.7).  Four waves (one a SIMD) instead of eight
-// were slower (55 at 2048 rows), reading the pivot row back from LDS instead
-// of by readlane too (50).
+// 4096 factored in 9.1 ms (12.7; 8.7 with the update below).  Four waves (one
+// a SIMD) instead of eight were slower (55 at 2048 rows), reading the pivot row
+// back from LDS instead of by readlane too (50).
 struct LuPanelShared {
   // per-wave candidates: the bits of |value| (0: none) and the physical row
   uint2 ckey[2][kLuWaves];
