@@ -413,7 +413,8 @@ int ozk_residual(const double* A, int64_t lda, const double* x, int64_t ldx,
  * the diagonal and U on and above it, and perm (device int32, n entries)
  * the row permutation (row i of P A is row perm[i] of A), the form
  * ozk_lu_solve_f32 takes.  The pivot of a column is its largest |value| on
- * or below the diagonal (the lowest row on ties).  flags is cleared first
+ * or below the diagonal (the lowest row on ties, earlier swaps applied, as
+ * LAPACK's getf2 chooses).  flags is cleared first
  * and receives OZK_FLAG_SINGULAR if a pivot is zero; as in LAPACK's getrf
  * the factorisation then completes and U has a zero on its diagonal.
  * n <= ozk_lu_factor_max_n(); larger n return OZK_ERR_UNSUPPORTED. */

@@ -76,7 +76,8 @@ __device__ __forceinline__ uint32_t lu_wave_reduce(uint32_t u) {
 // a SIMD) instead of eight were slower (55 at 2048 rows), reading the pivot row
 // back from LDS instead of by readlane too (50).
 struct LuPanelShared {
-  // per-wave candidates: the bits of |value| (0: none) and the physical row
+  // per-wave candidates: the bits of |value| (0: none), and the physical row
+  // with kLuTied if another row of the wave may equal it
   uint2 ckey[2][kLuWaves];
   float crow[2][kLuWaves][kLuSub];      //   and those rows' sub-panel registers
   float prow[kLuPanel][kLuSub];         // pivot rows: their own sub-panel's columns
@@ -84,9 +85,6 @@ struct LuPanelShared {
   float l10[kLuSub][kLuSub];            // second sub-panel's pivots: the first's columns
   float u01[kLuSub][kLuSub];            // U block right of the first sub-panel
   int prow_of[kLuPanel];                // physical pivot row of column j
-  int top[kLuPanel];                    // position of displaced row x < w
-  int displaced[kLuPanel];
-  uint32_t pivot_top;                   // bit x: row x < w is a pivot
   int pos[kLuWaves][64];
   float4 stage[kLuWaves][64 * kLuSub / 4];
 };
@@ -115,16 +113,32 @@ __device__ __forceinline__ float lu_readlane(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
+// Where the first `cols` columns' swaps leave physical row x, which must not be
+// a pivot of theirs (lanes with none: kLuNoRow): a row below `cols` went where its
+// column's pivot row was; if that is a row below `cols` too, where that row's
+// column's pivot was, and so on.  (Pivot rows differ, so the walk from a row
+// that is none never comes back to a row: it ends.)
+constexpr uint32_t kLuNoRow = ~0u, kLuTied = 1u << 31;
+__device__ __forceinline__ uint32_t lu_position(uint32_t x, uint32_t cols, const int* prow_of) {
+#pragma unroll 1
+  for (int k = 0; k < kLuPanel && x < cols; ++k) x = (uint32_t)prow_of[x];
+  return x;
+}
+
 // `steps` columns (panel columns dj0 ..) of a sub-panel over the rotating
 // registers 0 .. WD - 1: register 0 holds the active column, registers
 // WD - s .. WD - 1 the L entries of the s columns finished here.  lm[i]: all
 // ones while row slot i can still become a pivot, 0 for a pivot or no row;
-// field i of pcode receives 1 + the panel column a row becomes the pivot of.
-// The pivot is the candidate with the largest |value| (bit patterns: a NaN
-// wins); on ties the lowest wave, slot, lane.  Where every candidate is zero
-// the lowest row is taken, the column left as it is and OZK_FLAG_SINGULAR
-// raised.  fetch(pr, dj) starts the copy of pivot row pr's other sub-panel
-// into LDS (one wave).
+// 6-bit field i of pcode receives 1 + the panel column a row becomes the pivot
+// of.  The pivot is the candidate with the largest |value| (bit patterns: a NaN
+// wins); of equal ones the lowest in LAPACK's row order, its swaps so far
+// applied (lu_position): where several tie, the search is repeated among them
+// by position.  That path is almost never taken, but its presence costs random
+// matrices 1.4% (n = 4096: 8.63 -> 8.75 ms) to 2.6% (2048: 3.24 -> 3.33);
+// ordering inside the first search, before or behind its stores, cost 3 to 10%.
+// Where every candidate is zero the lowest row is taken, the column left as
+// it is and OZK_FLAG_SINGULAR raised.  fetch(pr, dj) starts the copy of pivot
+// row pr's other sub-panel into LDS (one wave).
 template <int S, int WD, class Fetch>
 __device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)[S],
                                            uint64_t& pcode, int dj0, int steps,
@@ -138,25 +152,30 @@ __device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)
     uint32_t u[S];
 #pragma unroll
     for (int i = 0; i < S; ++i) u[i] = __float_as_uint(r[i][0]) & lm[i] & 0x7fffffffu;
-    bool zero = false;  // every candidate is 0: choose by row
+    bool by_row = false;  // the candidates are those of equal magnitude, by position
     uint2 kv;
     float2 rv;
-    float pvl;
-    uint32_t best;
+    float pvl, rl;
+    int qw, pr;
 #pragma unroll 1
     for (;;) {
-      uint32_t mx = u[0];
+      uint32_t m1 = S > 1 ? u[S - 1] : 0u;  // of the slots above the first
 #pragma unroll
-      for (int i = 1; i < S; ++i) mx = max(mx, u[i]);
+      for (int i = 1; i < S - 1; ++i) m1 = max(m1, u[i]);
+      const uint32_t mx = max(u[0], m1);
       // the lane's slot (lowest of equals), while the wave's maximum forms
       int sel = S - 1;
 #pragma unroll
       for (int i = S - 2; i >= 0; --i) sel = u[i] == mx ? i : sel;
       const uint32_t wb = lu_wave_reduce<true>(mx);
-      const int hl = (int)__builtin_ctzll(__ballot(mx == wb));
+      // several lanes' candidates; or one lane's, whose first slot alone may
+      // hold a displaced row
+      const uint64_t tie = __ballot(mx == wb), both = S > 1 ? __ballot(u[0] == m1) : 0u;
+      const uint32_t tied = (tie & ((tie - 1u) | both)) != 0u ? kLuTied : 0u;
+      const int hl = (int)__builtin_ctzll(tie);
       const int slot = S > 1 ? __builtin_amdgcn_readlane(sel, hl) : 0;
       if (lane == hl) {
-        sh.ckey[par][wave] = make_uint2(wb, (uint32_t)(slot * kLuThreads + t));
+        sh.ckey[par][wave] = make_uint2(wb, (uint32_t)(slot * kLuThreads + t) | tied);
         static_for<0, S>([&](auto ic) {
           constexpr int i = decltype(ic)::value;
           if (i == slot) {
@@ -176,25 +195,33 @@ __device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)
       kv = sh.ckey[par][lane % kLuWaves];
       pvl = sh.crow[par][lane % kLuWaves][0];
       rv = *(const float2*)&sh.crow[par][lane / kLuWaves][k0];
-      best = kv.x;
+      uint32_t best = kv.x;
       best = max(best, lu_dpp<0xB1>(best));   // quad_perm [1, 0, 3, 2]
       best = max(best, lu_dpp<0x4E>(best));   // quad_perm [2, 3, 0, 1]
       best = max(best, lu_dpp<0x141>(best));  // half-row mirror: 8 lanes
       best = __builtin_amdgcn_readfirstlane(best);
-      if (best != 0u || zero) break;  // uniform over the workgroup
-      zero = true;
+      // LAPACK's getf2 scales by the pivot's reciprocal; below FLT_MIN, where
+      // that can overflow, pivot and column are scaled by 2^24 first (exact).
+      // Every lane inverts its candidate while the maximum forms (the empty
+      // asm keeps the compiler from doing it after the choice instead).
+      rl = 1.0f / (fabsf(pvl) < FLT_MIN ? pvl * 0x1p24f : pvl);
+      asm volatile("" : "+v"(rl));
+      const uint64_t won = __ballot(kv.x == best);
+      qw = (int)__builtin_ctzll(won);
+      pr = __builtin_amdgcn_readlane((int)kv.y, qw);
+      // one wave's only candidate (8 lanes read its key): uniform over the workgroup
+      if (__builtin_expect(
+              (__builtin_popcountll(won) == 64 / kLuWaves && pr >= 0) || by_row, 1))
+        break;
+      by_row = true;
+      const uint32_t at = lu_position(lm[0] ? (uint32_t)t : kLuNoRow, (uint32_t)dj, sh.prow_of);
 #pragma unroll
-      for (int i = 0; i < S; ++i) u[i] = (uint32_t)(INT_MAX - t - kLuThreads * i) & lm[i];
+      for (int i = 0; i < S; ++i)
+        u[i] = u[i] == best
+                   ? ((uint32_t)INT_MAX - (i ? (uint32_t)(t + kLuThreads * i) : at)) & lm[i]
+                   : 0u;
       __syncthreads();
     }
-    // LAPACK's getf2 scales by the pivot's reciprocal; below FLT_MIN, where
-    // that can overflow, pivot and column are scaled by 2^24 first (exact).
-    // Every lane inverts its candidate while the maximum forms (the empty
-    // asm keeps the compiler from doing it after the choice instead).
-    float rl = 1.0f / (fabsf(pvl) < FLT_MIN ? pvl * 0x1p24f : pvl);
-    asm volatile("" : "+v"(rl));
-    const int qw = (int)__builtin_ctzll(__ballot(kv.x == best));
-    const int pr = __builtin_amdgcn_readlane((int)kv.y, qw);
     const float pv = lu_readlane(pvl, qw);
     float rinv = lu_readlane(rl, qw);
     // the pivot row's columns right of the active one (0 for finished ones)
@@ -394,11 +421,11 @@ __device__ __forceinline__ void lu_update_rows(float (&b)[S][kLuSub], const floa
 // kLuThreads rows, w <= kLuPanel) and writes to maps the row permutation its
 // swaps make: maps[0] = w, then kLuPairs destination rows (absolute, -1 =
 // unused) and kLuPairs source rows.  Entries e < w are the diagonal
-// positions c + e; entry kLuPanel + j puts one of the rows c .. c + w - 1
-// that is no pivot at the place column j's pivot row came from.  Behind them
-// lies the panel's L block (rows c .. c + w - 1, kLuPanel x kLuPanel, zero on
-// and above the diagonal).  The first sub-panel's columns are stored with
-// their rows where they were; the row fix moves them with the columns left of the panel.
+// positions c + e; entry kLuPanel + x puts row c + x, x < w, if it is no
+// pivot, where the swaps moved it.  Behind them lies the panel's L block (rows
+// c .. c + w - 1, kLuPanel x kLuPanel, zero on and above the diagonal).  The
+// first sub-panel's columns are stored with their rows where they were; the
+// row fix moves them with the columns left of the panel.
 //
 // Up to S = kLuPreload row slots the second sub-panel's loads are issued
 // before the first is factored; above, the registers hold them in two halves
@@ -417,7 +444,6 @@ __global__ __launch_bounds__(kLuThreads) void lu_panel_kernel(float* __restrict_
   const int m = n - c;
   const int w0 = w < kLuSub ? w : kLuSub, w1 = w - w0;
   float* const P = A + (int64_t)c * lda + c;
-  if (t == 0) sh.pivot_top = 0u;  // (ordered by the columns' barriers)
   uint64_t pcode = 0u;
   uint32_t lm[S];
 #pragma unroll
@@ -487,31 +513,16 @@ __global__ __launch_bounds__(kLuThreads) void lu_panel_kernel(float* __restrict_
     if (wave == kLuWaves - 1) wait_vm<0>();
   }
   __syncthreads();  // prow_of, prow and l10 final
-  // The permutation: position j takes pivot row j; the rows below w that are
-  // no pivots, in order, take the places the pivots from w on leave.
-  const bool col = t < w;
-  const int pj = col ? sh.prow_of[t] : -1;
-  if (wave == 0) {
-    if (col && pj < w) atomicOr(&sh.pivot_top, 1u << pj);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    const uint32_t piv = sh.pivot_top;
-    if (col) sh.top[t] = t;
-    if (col && !((piv >> t) & 1u))
-      sh.displaced[__popc(~piv & ((1u << t) - 1u))] = t;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    const uint64_t vac = __ballot(col && pj >= w);
-    int dst = -1, src = 0;
-    if (col && pj >= w) {
-      dst = pj;
-      src = sh.displaced[__popcll(vac & ((1ull << t) - 1ull))];
-      sh.top[src] = dst;
-    }
-    if (t < kLuPanel) {
-      maps[1 + t] = col ? c + t : -1;
-      maps[1 + kLuPairs + t] = c + (col ? pj : 0);
-      maps[1 + kLuPanel + t] = dst >= 0 ? c + dst : -1;
-      maps[1 + kLuPairs + kLuPanel + t] = c + src;
-    }
+  // The permutation: position j takes pivot row j, and a row below w that is
+  // no pivot goes where the swaps left it.
+  const bool moves = t < w && (pcode & 63u) == 0u;
+  const int top = (int)lu_position(moves ? (uint32_t)t : kLuNoRow, (uint32_t)w, sh.prow_of);
+  if (t < kLuPanel) {
+    const bool col = t < w;
+    maps[1 + t] = col ? c + t : -1;
+    maps[1 + kLuPairs + t] = c + (col ? sh.prow_of[t] : 0);
+    maps[1 + kLuPanel + t] = moves ? c + top : -1;
+    maps[1 + kLuPairs + kLuPanel + t] = c + (moves ? t : 0);
     if (t == 0) maps[0] = w;
   }
   float* const L = (float*)(maps + kLuMapInts);
@@ -525,12 +536,11 @@ __global__ __launch_bounds__(kLuThreads) void lu_panel_kernel(float* __restrict_
     L[e] = v;
   }
   if (w1 > 0) {
-    __syncthreads();  // top final
     lu_store_rows<VEC>(b, P, lda, kLuSub, w1, sh, [&](int i) {
       const int ph = t + i * kLuThreads, code = (int)((pcode >> (6 * i)) & 63u);
       if (ph >= m || (code > 0 && code <= kLuSub)) return -1;  // U01's rows are stored above
       if (code > 0) return code - 1;
-      return ph < w ? sh.top[ph < kLuPanel ? ph : 0] : ph;
+      return ph < w ? top : ph;
     });
   }
 }

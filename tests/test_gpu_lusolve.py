@@ -268,7 +268,8 @@ def check_lu(A32, F, perm):
 # 512 rows a register slot: first panels of exactly 1, 2 and 5 slots and one
 # row more, last panels of 1, 15, 16, 17 and 31 columns, 16-byte rows or not
 @pytest.mark.parametrize("n,pad", [(15, 1), (31, 0), (49, 3), (512, 0), (513, 3), (1024, 0),
-                                   (1039, 1), (1040, 0), (2560, 0), (2561, 3)])
+                                   (1039, 1), (1040, 0), (2560, 0), (2561, 3),
+                                   (3073, 0), (3585, 2), (4095, 0)])
 def test_lu_factor_row_slot_edges(ozk, n, pad):
     A32 = np.random.RandomState(300 + n).randn(n, n).astype(np.float32)
     case(f"ozk_lu_factor_f32 n={n} lda=n+{pad} (slot and panel edges)")
@@ -296,6 +297,60 @@ def test_lu_factor_subnormal_pivots_and_ties(ozk):
     U = np.triu(F.astype(np.float64))
     err = np.abs(A32.astype(np.float64)[perm] - L @ U)[:, 5].max()
     assert err <= n * 2.0 ** -149, err
+
+
+def getf2(A32):
+    """Unblocked partial pivoting as LAPACK's getf2 does it, the first of
+    equal magnitudes in the present row order, on entries whose elimination
+    is exact in FP32 (any order of the updates gives the same bits):
+    (factor, perm)."""
+    F = A32.copy()
+    n = F.shape[0]
+    perm = np.arange(n, dtype=np.int32)
+    for j in range(n):
+        p = j + int(np.argmax(np.abs(F[j:, j])))
+        F[[j, p]] = F[[p, j]]
+        perm[[j, p]] = perm[[p, j]]
+        if F[j, j] == 0:
+            continue
+        F[j + 1:, j] /= F[j, j]
+        r = j + 1 + np.flatnonzero(F[j + 1:, j])
+        F[r, j + 1:] -= np.outer(F[r, j], F[j, j + 1:])
+    return F, perm
+
+
+def network_matrix(n, rng):
+    """A network matrix: column e holds the signed edges of one tree's path
+    between the ends of edge e of another tree.  It is totally unimodular and
+    nonsingular: every entry at every step of its elimination is 0 or +-1, so
+    all candidates of every column tie and all arithmetic is exact."""
+    up = [rng.randint(max(0, v - 8), v, size=2) for v in range(1, n + 1)]  # both trees' parents
+    path = np.zeros((n + 1, n), np.float32)  # first tree: edges from vertex v to the root
+    for v in range(1, n + 1):
+        path[v] = path[up[v - 1][0]]
+        path[v, v - 1] += 1
+    name = rng.permutation(n + 1)  # of the second tree's vertices in the first
+    A = np.stack([path[name[v]] - path[name[up[v - 1][1]]] for v in range(1, n + 1)], axis=1)
+    return np.ascontiguousarray(A[rng.permutation(n)][:, rng.permutation(n)])
+
+
+@pytest.mark.parametrize("n,pad,zeros", [(70, 0, 0), (300, 1, 0), (512, 0, 9), (700, 0, 0),
+                                         (1301, 0, 0), (1301, 3, 40), (2600, 0, 0)])
+def test_lu_factor_takes_the_lowest_row_of_equal_pivots(ozk, n, pad, zeros):
+    """Ties between all lanes, waves and row slots, with rows displaced by
+    earlier swaps among them, and (zeros) columns without a nonzero
+    candidate: the same permutation and factor as getf2, bit for bit."""
+    from ozaki_jax_amd import _lib
+    rng = np.random.RandomState(500 + n)
+    A32 = network_matrix(n, rng)
+    if zeros:  # repeated columns
+        A32[:, rng.choice(n // 2, zeros, False) + n // 2] = A32[:, :zeros]
+    Fr, pr = getf2(A32)
+    case(f"ozk_lu_factor_f32 n={n} lda=n+{pad} all pivots tied, {zeros} repeated columns")
+    F, perm, flags = gpu_factor(A32, pad)
+    assert bool(flags & _lib.OZK_FLAG_SINGULAR) == bool(zeros)
+    assert np.array_equal(perm, pr)
+    assert np.array_equal(F, Fr)
 
 
 def test_lu_factor_singular_flag(ozk):
