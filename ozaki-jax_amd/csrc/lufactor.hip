@@ -200,11 +200,10 @@ __device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)
       best = max(best, lu_dpp<0x4E>(best));   // quad_perm [2, 3, 0, 1]
       best = max(best, lu_dpp<0x141>(best));  // half-row mirror: 8 lanes
       best = __builtin_amdgcn_readfirstlane(best);
-      // LAPACK's getf2 scales by the pivot's reciprocal; below FLT_MIN, where
-      // that can overflow, pivot and column are scaled by 2^24 first (exact).
-      // Every lane inverts its candidate while the maximum forms (the empty
-      // asm keeps the compiler from doing it after the choice instead).
-      rl = 1.0f / (fabsf(pvl) < FLT_MIN ? pvl * 0x1p24f : pvl);
+      // LAPACK's getf2 scales by the pivot's reciprocal.  Every lane inverts
+      // its candidate while the maximum forms (the empty asm keeps the
+      // compiler from doing it after the choice instead).
+      rl = 1.0f / pvl;
       asm volatile("" : "+v"(rl));
       const uint64_t won = __ballot(kv.x == best);
       qw = (int)__builtin_ctzll(won);
@@ -250,9 +249,12 @@ __device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)
       if (pv == 0.0f) {
         rinv = 0.0f;
         if (t == 0) atomicOr(status, OZK_FLAG_SINGULAR);
-      } else {  // (the pivot row itself is out of lm by now)
+      } else {
+        // the reciprocal can overflow: getf2 divides here, one rounding a
+        // multiplier (the pivot row itself is out of lm by now)
+        rinv = 1.0f;
 #pragma unroll
-        for (int i = 0; i < S; ++i) r[i][0] = lm[i] ? r[i][0] * 0x1p24f : r[i][0];
+        for (int i = 0; i < S; ++i) r[i][0] = lm[i] ? r[i][0] / pv : r[i][0];
       }
     }
 #pragma unroll

@@ -353,6 +353,26 @@ def test_lu_factor_takes_the_lowest_row_of_equal_pivots(ozk, n, pad, zeros):
     assert np.array_equal(F, Fr)
 
 
+@pytest.mark.parametrize("n,pad,col", [(70, 0, 0), (600, 0, 20), (600, 1, 33), (2600, 0, 5)])
+def test_lu_factor_divides_by_a_subnormal_pivot(ozk, n, pad, col):
+    """Below FLT_MIN LAPACK's getf2 divides by the pivot, one rounding a
+    multiplier (scaled reciprocals round twice: up to half of these
+    multipliers would differ).  The columns before `col` are unit vectors,
+    so that column's multipliers are quotients of entries of A."""
+    rng = np.random.RandomState(700 + n + col)
+    A32 = rng.randn(n, n).astype(np.float32)
+    A32[:, :col] = 0.0
+    A32[np.arange(col), np.arange(col)] = 4.0
+    x = (rng.randint(-8388607, 8388608, n) * 2.0 ** -149).astype(np.float32)
+    A32[col:, col] = x[col:]
+    case(f"ozk_lu_factor_f32 n={n} lda=n+{pad} subnormal column {col}")
+    F, perm, flags = gpu_factor(A32, pad)
+    assert flags == 0
+    p = x[perm[col]]
+    assert 0 < abs(p) < np.finfo(np.float32).tiny and abs(p) == np.abs(x[col:]).max()
+    assert np.array_equal(F[col + 1:, col], x[perm[col + 1:]] / p)
+
+
 def test_lu_factor_singular_flag(ozk):
     from ozaki_jax_amd import _lib
     rng = np.random.RandomState(7)
