@@ -134,7 +134,7 @@ __device__ __forceinline__ uint32_t lu_position(uint32_t x, uint32_t cols, const
 // wins); of equal ones the lowest in LAPACK's row order, its swaps so far
 // applied (lu_position): where several tie, the search is repeated among them
 // by position.  That path is almost never taken, but its presence costs random
-// matrices 1.4% (n = 4096: 8.63 -> 8.75 ms) to 2.6% (2048: 3.24 -> 3.33);
+// matrices 0.5% (n = 4096: 8.66 -> 8.71 ms) to 1.6% (2048: 3.25 -> 3.30);
 // ordering inside the first search, before or behind its stores, cost 3 to 10%.
 // Where every candidate is zero the lowest row is taken, the column left as
 // it is and OZK_FLAG_SINGULAR raised.  fetch(pr, dj) starts the copy of pivot
@@ -247,7 +247,10 @@ __device__ __forceinline__ void lu_columns(float (&r)[S][kLuSub], uint32_t (&lm)
     }
     if (fabsf(pv) < FLT_MIN) {  // uniform
       if (pv == 0.0f) {
+        // no update: 0 * p would carry an infinity of its row to all others
         rinv = 0.0f;
+#pragma unroll
+        for (int k = 1; k < WD; ++k) p[k] = 0.0f;
         if (t == 0) atomicOr(status, OZK_FLAG_SINGULAR);
       } else {
         // the reciprocal can overflow: getf2 divides here, one rounding a

@@ -373,6 +373,21 @@ def test_lu_factor_divides_by_a_subnormal_pivot(ozk, n, pad, col):
     assert np.array_equal(F[col + 1:, col], x[perm[col + 1:]] / p)
 
 
+def test_lu_factor_zero_pivot_leaves_the_other_rows(ozk):
+    """A column without a nonzero candidate is passed over: an infinity in
+    the row at its diagonal does not reach the rows below."""
+    from ozaki_jax_amd import _lib
+    A32 = np.random.RandomState(11).randn(12, 12).astype(np.float32)
+    want, pw, _ = gpu_factor(np.ascontiguousarray(A32[1:, 1:]))
+    A32[:, 0] = 0.0
+    A32[0, 7] = np.inf
+    case("ozk_lu_factor_f32 zero column, infinity in the row at its diagonal")
+    F, perm, flags = gpu_factor(A32)
+    assert flags & _lib.OZK_FLAG_SINGULAR
+    assert perm[0] == 0 and np.array_equal(perm[1:], pw + 1)
+    assert np.array_equal(F[1:, 1:], want)
+
+
 def test_lu_factor_singular_flag(ozk):
     from ozaki_jax_amd import _lib
     rng = np.random.RandomState(7)
