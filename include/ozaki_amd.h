@@ -343,7 +343,8 @@ int ozk_wait_flag_word(const uint32_t* host_word, void* stream, uint32_t* flags)
  * copies are queued, to the host when the array is complete.  It waits for a
  * slot's event before it uses the slot, so calls may follow one another at
  * once.
- * Pinned memory serves one call at a time. */
+ * Pinned memory serves one call at a time.  Both return OZK_ERR_HIP on a
+ * stream that is being captured, with nothing recorded. */
 int ozk_copy_to_host(void* host, const void* dev, size_t bytes, void* staging,
                      size_t staging_bytes, uint32_t* flags,
                      uint32_t* zero_counts, int threads, void* stream);

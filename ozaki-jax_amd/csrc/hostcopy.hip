@@ -336,6 +336,16 @@ static int copy_slots(bool down, void* dev, void* host, size_t bytes, void* stag
   return OZK_OK;
 }
 
+// Pinned memory is used again by later calls and a result is waited for, so
+// neither copy can be part of a captured graph.
+static int refuse_capture(hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  OZK_HIP(hipStreamIsCapturing(st, &cap));
+  if (cap == hipStreamCaptureStatusNone) return OZK_OK;
+  set_error("a staged copy cannot be captured");
+  return OZK_ERR_HIP;
+}
+
 }  // namespace ozk
 
 using namespace ozk;
@@ -350,12 +360,8 @@ int ozk_copy_to_host(void* host, const void* dev, size_t bytes, void* staging,
                 "staged copy: invalid pinned memory of %zu bytes", staging_bytes);
   if (bytes == 0) return OZK_OK;
   OZK_CHECK_ARG(host && dev && staging && flags && zero_counts, "null pointer");
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  OZK_HIP(hipStreamIsCapturing((hipStream_t)stream, &cap));
-  if (cap != hipStreamCaptureStatusNone) {
-    set_error("a copy to the host under stream capture cannot be waited for");
-    return OZK_ERR_HIP;
-  }
+  const int rc = refuse_capture((hipStream_t)stream);
+  if (rc) return rc;
   try {
     return copy_out(host, dev, bytes, staging, staging_bytes, flags, zero_counts, threads,
                     (hipStream_t)stream);
@@ -374,6 +380,8 @@ int ozk_copy_slots(int down, void* dev, void* host, size_t bytes, void* staging,
                 "staged copy: invalid ring (%d slots of %zu bytes)", slots, slot_bytes);
   if (bytes == 0) return OZK_OK;
   OZK_CHECK_ARG(host && dev && staging && events, "null pointer");
+  const int rc = refuse_capture((hipStream_t)stream);
+  if (rc) return rc;
   try {
     return copy_slots(down != 0, dev, host, bytes, staging, slot_bytes, slots, first, events,
                       threads, (hipStream_t)stream);
