@@ -152,22 +152,24 @@ _STAGE_CHUNK = 64 << 20
 
 
 class _Slots:
-    """Pinned slots with an event each (ozk_copy_slots).  One transfer at a
-    time (a lock)."""
+    """Pinned slots with an event each (ozk_copy_slots, which sees to it that
+    transfers of several threads do not meet).  The lock hands out the slot a
+    transfer starts at."""
 
     def __init__(self, rt, slot, slots):
         self.slot, self.slots, self.first = int(slot), int(slots), 0
         self.buf = rt.host_malloc(self.slot * self.slots)
         self.ev = (ctypes.c_void_p * self.slots)(*[rt.event() for _ in range(self.slots)])
+        self.owners = (ctypes.c_void_p * self.slots)()
         self.lock = threading.Lock()
 
     def copy(self, down, dev_ptr, host, threads, stream):
         with self.lock:
             first = self.first
             self.first = (first + -(-host.nbytes // self.slot)) % self.slots
-            _lib.check(_lib.load().ozk_copy_slots(
-                down, dev_ptr, host.ctypes.data, host.nbytes, self.buf, self.slot, self.slots,
-                first, self.ev, threads, stream))
+        _lib.check(_lib.load().ozk_copy_slots(
+            down, dev_ptr, host.ctypes.data, host.nbytes, self.buf, self.slot, self.slots,
+            first, self.ev, self.owners, threads, stream))
 
     def release(self, h):
         h.hipHostFree(self.buf)
@@ -179,8 +181,8 @@ class _Stager:
     """Pinned memory of the library's staged copies, allocated once per device
     and kept for the process: slots for the way up, as much memory with a
     flag word and a device counter per 512 KiB for the way down
-    (ozk_copy_to_host), and larger slots for large transfers either way.  One
-    transfer at a time in each (a lock)."""
+    (ozk_copy_to_host), and larger slots for large transfers either way.  A
+    transfer that finds its memory in use by another thread's goes without."""
 
     def __init__(self, rt, slot=_SLOT, slots=_SLOTS):
         self.rt, self.size = rt, int(slot) * int(slots)
@@ -217,10 +219,9 @@ class _Stager:
         if out.nbytes > _SLOT * _SLOTS:
             self._big().copy(1, dev_ptr, out, self._threads(out.nbytes), stream)
             return
-        with self.lock:
-            _lib.check(_lib.load().ozk_copy_to_host(
-                out.ctypes.data, dev_ptr, out.nbytes, self.down, self.size, self.flags,
-                self.counts, self._threads(out.nbytes), stream))
+        _lib.check(_lib.load().ozk_copy_to_host(
+            out.ctypes.data, dev_ptr, out.nbytes, self.down, self.size, self.flags,
+            self.counts, self._threads(out.nbytes), stream))
 
     def release(self, h):
         self.up.release(h)

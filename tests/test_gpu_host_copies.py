@@ -31,7 +31,7 @@ def test_slots_refuse_a_captured_stream(ozk, mode):
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g, capture_error_mode=mode):
             rc = lib.ozk_copy_slots(down, t.data_ptr(), a.ctypes.data, a.nbytes, st.up.buf,
-                                    st.up.slot, st.up.slots, 0, st.up.ev, 2,
+                                    st.up.slot, st.up.slots, 0, st.up.ev, st.up.owners, 2,
                                     torch.cuda.current_stream().cuda_stream)
             err = ctypes.string_at(lib.ozk_last_error())
             t.zero_()  # the capture itself goes on
@@ -60,3 +60,61 @@ def test_residual_with_numpy_operands_refuses_capture(ozk):
             ozk.residual(A, x, b, mode="ozaki")
         x.zero_()
     assert torch.equal(ozk.residual(A, x, b, mode="ozaki"), want)
+
+
+def _busy(stream, seconds):
+    """A kernel of about this long on `stream` (one spinning workgroup), and
+    the event behind it."""
+    import torch
+    with torch.cuda.stream(stream):
+        e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        e0.record()
+        torch.cuda._sleep(1000000)
+        e1.record()
+        e1.synchronize()
+        cycles = int(1000000 * seconds * 1e3 / e0.elapsed_time(e1))
+        done = torch.cuda.Event()
+        torch.cuda._sleep(cycles)
+        done.record()
+    return done
+
+
+@pytest.mark.parametrize("way,mib", [("down", 4), ("down", 48), ("up", 32), ("up", 130)])
+def test_copies_do_not_wait_for_another_threads_stream(ozk, way, mib):
+    """One thread copies on a stream that is busy for a second; a copy of
+    another thread, on an idle stream through the same pinned memory, is done
+    long before that."""
+    import threading
+    import torch
+    from ozaki_jax_amd import _device as D
+    n = (mib << 20) // 8
+    dev = torch.device("cuda", torch.cuda.current_device())
+    rng = np.random.RandomState(mib)
+    a = [rng.randn(n // 1024, 1024) for _ in range(2)]
+    t = [torch.from_numpy(v).cuda() for v in a]
+    for i in range(2):  # the pinned memory of this size is there
+        assert np.array_equal(D._torch_to_numpy(D._numpy_to_torch(a[i], dev)), a[i])
+    busy = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    case(f"{way} {mib} MiB beside a busy stream")
+    done = _busy(busy, 1.0)
+    got, inside = {}, threading.Event()
+
+    def first():
+        with torch.cuda.stream(busy):
+            inside.set()
+            got[0] = D._torch_to_numpy(t[0]) if way == "down" else D._numpy_to_torch(a[0], dev)
+
+    th = threading.Thread(target=first)
+    th.start()
+    inside.wait()
+    threading.Event().wait(0.2)  # the first thread's copy has begun
+    got[1] = D._torch_to_numpy(t[1]) if way == "down" else D._numpy_to_torch(a[1], dev)
+    if way == "up":
+        torch.cuda.current_stream().synchronize()
+    early = not done.query()
+    th.join()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert np.array_equal(got[i] if way == "down" else got[i].cpu().numpy(), a[i])
+    assert early, "the copy waited for the other thread's stream"
