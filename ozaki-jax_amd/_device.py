@@ -85,8 +85,8 @@ class FlagWords:
     """A zeroed device word, which collects a call's flags, and the pinned
     host word that the call's GEMM publishes them to.  run(call, stream) makes
     the call and returns its flags once they are published; the product may
-    still be queued then.  After an error the pair is not used again, since
-    what was queued may still write it."""
+    still be queued then.  After a failure on the GPU the pair is not used
+    again, since what was queued may still write it."""
 
     def __init__(self, device):
         rt = _hip._rt()
@@ -108,18 +108,24 @@ class FlagWords:
     def run(self, call, stream):
         lib = _lib.load()
         self.word.value = 0
-        _lib.check(call(self.dev, self.host))
+        rc = call(self.dev, self.host)
+        if rc < 0 and rc != _lib.OZK_ERR_HIP:  # refused before anything was queued
+            self.give_back()
+        _lib.check(rc)
         fl = ctypes.c_uint32()
         _lib.check(lib.ozk_wait_flag_word(self.host, stream, ctypes.byref(fl)))
+        self.give_back()
+        return fl.value
+
+    def give_back(self):
         with _early_lock:
             free = _flag_words_free.setdefault(self.device, [])
             if len(free) < _FLAG_WORDS_KEPT:
                 free.append(self)
-                return fl.value
+                return
         rt = _hip._rt()
         rt.free(self.dev)
         rt.host_free(self.host)
-        return fl.value
 
 
 class _TorchFamily:

@@ -513,7 +513,7 @@ static int matmul_call(const double* A, int64_t lda, const double* B, int64_t ld
                        double* C, int64_t ldc, int64_t N, int64_t K, int64_t M,
                        int pipeline, int n_hi, int n_lo, int order, void* workspace,
                        size_t workspace_bytes, uint32_t* flags, uint32_t* host_flags,
-                       void* event, void* stream, FlagPub pub = {}) {
+                       void* event, void* stream, FlagPub pub = {}, bool* queued = nullptr) {
   clear_error();
   hipStream_t st = (hipStream_t)stream;
   const int pipe_arg = pipeline;
@@ -548,6 +548,7 @@ static int matmul_call(const double* A, int64_t lda, const double* B, int64_t ld
   size_t dyn_bytes;
   const size_t dyn_off = gemm_dyn_counters(N, M, pipeline, n_hi, n_lo, order, &dyn_bytes);
   zero.add((char*)gws + dyn_off, dyn_bytes);
+  if (queued) *queued = true;
   if (pipeline == OZK_PIPE_ONDEVICE) {
     rho = rho_generic(K, 24);
     if (!i8 && extract_pair_f32(A, lda, B, ldb, N, K, M, rho, n_hi, n_lo, sa.s, sa.e, sb.s,
@@ -605,8 +606,11 @@ int ozk_matmul_flag_word(const double* A, int64_t lda, const double* B, int64_t 
   FlagPub pub;
   pub.flags = zero_flags;
   pub.host = host_word;
-  return matmul_call(A, lda, B, ldb, C, ldc, N, K, M, pipeline, n_hi, n_lo, order,
-                     workspace, workspace_bytes, zero_flags, nullptr, nullptr, stream, pub);
+  bool queued = false;
+  const int rc =
+      matmul_call(A, lda, B, ldb, C, ldc, N, K, M, pipeline, n_hi, n_lo, order, workspace,
+                  workspace_bytes, zero_flags, nullptr, nullptr, stream, pub, &queued);
+  return rc < 0 && queued ? OZK_ERR_HIP : rc;
 }
 
 int ozk_wait_flag_word(const uint32_t* host_word, void* stream, uint32_t* flags) {
@@ -668,7 +672,7 @@ size_t ozk_gram_workspace_bytes(int64_t rows, int64_t cols, int n_hi,
 static int gram_call(const double* A, int64_t lda, int64_t rows, int64_t cols, int n_hi,
                      int n_lo, double* G, int64_t ldg, void* workspace,
                      size_t workspace_bytes, uint32_t* flags, uint32_t* host_flags,
-                     void* event, void* stream, FlagPub pub = {}) {
+                     void* event, void* stream, FlagPub pub = {}, bool* queued = nullptr) {
   clear_error();
   hipStream_t st = (hipStream_t)stream;
   int rc = check_counts(OZK_PIPE_ONDEVICE, n_hi, n_lo);
@@ -699,6 +703,7 @@ static int gram_call(const double* A, int64_t lda, int64_t rows, int64_t cols, i
   const size_t dyn_off =
       gemm_dyn_counters(cols, cols, OZK_PIPE_ONDEVICE, n_hi, n_lo, OZK_ORDER_2SUM, &dyn_bytes);
   zero.add((char*)gws + dyn_off, dyn_bytes);
+  if (queued) *queued = true;
   if ((rc = extract<float>(A, rows, cols, lda, 1, rho, n_hi, n_lo, s.s, s.e,
                            flags, tws, extract_workspace_bytes(rows, cols, 1, false), st,
                            i8, s.sum, zero)))
@@ -745,8 +750,10 @@ int ozk_gram_flag_word(const double* A, int64_t lda, int64_t rows, int64_t cols,
   FlagPub pub;
   pub.flags = zero_flags;
   pub.host = host_word;
-  return gram_call(A, lda, rows, cols, n_hi, n_lo, G, ldg, workspace, workspace_bytes,
-                   zero_flags, nullptr, nullptr, stream, pub);
+  bool queued = false;
+  const int rc = gram_call(A, lda, rows, cols, n_hi, n_lo, G, ldg, workspace, workspace_bytes,
+                           zero_flags, nullptr, nullptr, stream, pub, &queued);
+  return rc < 0 && queued ? OZK_ERR_HIP : rc;
 }
 
 // Residual workspace.  Up to 4 right-hand sides with K <= 16384 (presets

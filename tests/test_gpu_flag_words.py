@@ -140,3 +140,24 @@ def test_concurrent_calls_have_words_of_their_own(ozk):
     for t in ts:
         t.join()
     assert not wrong, wrong
+
+
+def test_rejected_calls_give_their_words_back(ozk, monkeypatch):
+    """A call that the library refuses before anything is queued leaves its
+    words usable: no allocation per rejected call."""
+    import torch
+    from ozaki_jax_amd import _device as D, _hip
+    monkeypatch.setattr(D, "_flag_words_free", {})
+    A = torch.from_numpy(np.random.RandomState(0).randn(64, 300)).to("cuda")
+    want = ozk.matmul(A, A.T.contiguous(), pipeline="ondevice")  # one pair is there
+    rt, got = _hip._rt(), []
+    host_malloc = rt.host_malloc
+    monkeypatch.setattr(rt, "host_malloc", lambda n: (got.append(n), host_malloc(n))[1])
+    case("products and Gram matrices with slice counts that are refused")
+    for _ in range(5):
+        with pytest.raises(ValueError):
+            ozk.matmul(A, A.T.contiguous(), pipeline="ondevice", precision=(40, 1))
+        with pytest.raises(ValueError):
+            ozk.gram(A, precision=(40, 1), mode="ozaki")
+    assert torch.equal(ozk.matmul(A, A.T.contiguous(), pipeline="ondevice"), want)
+    assert not got
