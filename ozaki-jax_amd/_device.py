@@ -120,12 +120,33 @@ class FlagWords:
     def give_back(self):
         with _early_lock:
             free = _flag_words_free.setdefault(self.device, [])
+            if self in free:  # run again by who made it
+                return
             if len(free) < _FLAG_WORDS_KEPT:
                 free.append(self)
                 return
         rt = _hip._rt()
         rt.free(self.dev)
         rt.host_free(self.host)
+
+
+def _release_words(h):
+    """Frees the kept words and events of all devices (at exit)."""
+    with _early_lock:
+        words = [w for free in _flag_words_free.values() for w in free]
+        pairs = [p for free in _early_free.values() for p in free]
+        _flag_words_free.clear()
+        for free in _early_free.values():  # (a pair in use goes back to its list)
+            free.clear()
+    for w in words:
+        h.hipFree(w.dev)
+        h.hipHostFree(w.host)
+    for word, ev in pairs:
+        h.hipHostFree(word)
+        h.hipEventDestroy(ev)
+
+
+_hip._exit_hooks.append(_release_words)
 
 
 class _TorchFamily:

@@ -464,12 +464,15 @@ def _rt():
     return _get("rt", _Runtime)
 
 
+_exit_hooks = []  # called with the runtime's entry points once the device is idle
+
+
 def _release_at_exit():
     """At interpreter exit, before the runtime's own teardown: let queued
-    work end, then release what this module holds in the runtime (the
+    work end, then release what this package holds in the runtime (the
     staging buffers and their events, the rocBLAS handle, the compute stream,
-    the pool's cached blocks), so that none of it is left for the runtime's
-    static destructors.  The runtime and the pool stay: blocks that arrays
+    the pool's cached blocks, and through _exit_hooks what other modules keep),
+    so that none of it is left for the runtime's static destructors.  The runtime and the pool stay: blocks that arrays
     release later are freed at once.  Errors are ignored: the runtime may be
     unusable by then."""
     with _state_lock:
@@ -483,6 +486,8 @@ def _release_at_exit():
     h = rt.h
     try:
         h.hipDeviceSynchronize()
+        for hook in _exit_hooks:
+            hook(h)
         for stager in st.values():
             if isinstance(stager, _Stager):
                 stager.release(h)

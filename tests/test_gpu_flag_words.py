@@ -161,3 +161,22 @@ def test_rejected_calls_give_their_words_back(ozk, monkeypatch):
             ozk.gram(A, precision=(40, 1), mode="ozaki")
     assert torch.equal(ozk.matmul(A, A.T.contiguous(), pipeline="ondevice"), want)
     assert not got
+
+
+def test_kept_words_are_released(ozk):
+    """What is kept between calls is released by the exit hook, and calls
+    after that allocate anew."""
+    import torch
+    from ozaki_jax_amd import _device as D, _hip
+    A = torch.from_numpy(np.random.RandomState(0).randn(64, 300)).to("cuda")
+    want = ozk.gram(A, mode="ozaki")
+    word, ev, read = D._TorchFamily().early_flags()
+    _hip._rt().record(ev)
+    read()
+    torch.cuda.synchronize()
+    assert any(D._flag_words_free.values()) and any(D._early_free.values())
+    case("release of the kept words")
+    for hook in _hip._exit_hooks:
+        hook(_hip._rt().h)
+    assert not any(D._flag_words_free.values()) and not any(D._early_free.values())
+    assert torch.equal(ozk.gram(A, mode="ozaki"), want)
