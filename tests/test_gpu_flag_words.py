@@ -13,6 +13,17 @@ def case(msg):
     print(f"[case] {msg}", flush=True)
 
 
+def device_word(words):
+    """The device word once the device is idle."""
+    import ctypes
+    import torch
+    from ozaki_jax_amd import _hip
+    torch.cuda.synchronize()
+    v = ctypes.c_uint32(7)
+    _hip._rt().copy(ctypes.addressof(v), words.dev, 4, _hip._D2H)
+    return v.value
+
+
 # (shape, pipeline, n_hi, n_lo, order, input): orders 0 2Sum, 1 FP64 block,
 # 2 host; (6, 1) rectangle sweeps, (9, 1) the pairwise kernel
 CASES = [((130, 8192, 70), 0, 4, 1, 0, None), ((130, 8192, 70), 0, 4, 1, 0, "nan"),
@@ -55,6 +66,12 @@ def test_flag_word_matches_matmul(ozk, shape, pipe, nh, nl, order, kind):
         got = words.run(lambda d, h: lib.ozk_matmul_flag_word(*args(C2), d, h, D.stream_handle()),
                         D.stream_handle())
         assert got == want
+        assert device_word(words) == 0
+    if kind:  # finite inputs on the same words: no flag is left over
+        At.copy_(torch.from_numpy(np.where(np.isfinite(A) & (np.abs(A) < 1e9), A, 1.0)))
+        C3 = torch.empty_like(C2)
+        assert words.run(lambda d, h: lib.ozk_matmul_flag_word(*args(C3), d, h, D.stream_handle()),
+                         D.stream_handle()) == 0
     torch.cuda.synchronize()
     assert bool(want & _lib.OZK_FLAG_NONFINITE) == (kind == "nan")
     assert np.array_equal(C1.cpu().numpy(), C2.cpu().numpy(), equal_nan=True)
@@ -82,10 +99,10 @@ def test_gram_flag_word_matches_gram(ozk, rows, cols, nh, nl, kind):
 
     case(f"ozk_gram_flag_word ({rows},{cols}) ({nh},{nl}) {kind}")
     _lib.check(lib.ozk_gram(*args(0), f.data_ptr(), D.stream_handle()))
-    got = D.FlagWords(0).run(lambda d, h: lib.ozk_gram_flag_word(*args(1), d, h,
-                                                                 D.stream_handle()),
-                             D.stream_handle())
-    torch.cuda.synchronize()
+    words = D.FlagWords(0)
+    got = words.run(lambda d, h: lib.ozk_gram_flag_word(*args(1), d, h, D.stream_handle()),
+                    D.stream_handle())
+    assert device_word(words) == 0
     assert got == int(f.item()) & 0xffffffff
     assert bool(got & _lib.OZK_FLAG_NONFINITE) == (kind == "nan")
     assert np.array_equal(G[0].cpu().numpy(), G[1].cpu().numpy(), equal_nan=True)
