@@ -150,7 +150,10 @@ _hip._exit_hooks.append(_release_words)
 
 
 class _TorchFamily:
-    """Torch tensors on torch's current device and stream."""
+    """Torch tensors on torch's current device and stream.  stream_ordered:
+    results may be returned while their kernels are queued."""
+
+    stream_ordered = True
 
     def __init__(self):
         if torch is None or not torch.cuda.is_available():
@@ -198,11 +201,11 @@ class _TorchFamily:
         return torch.zeros(shape, dtype=_TORCH_DTYPES[np.dtype(dtype)], device=self.dev)
 
     def early_flags(self):
-        """(host word, event, read) for ozk_matmul_early_flags: a pinned
-        host word and a HIP event of this device, taken from a shared free
-        list, and read() waiting for the event, returning the word and giving
-        the pair back.  The product stays ordered on the current stream, as
-        torch's own results are."""
+        """(host word, event, read) for callers of ozk_matmul_early_flags and
+        ozk_gram_early_flags: a pinned host word and a HIP event of this
+        device, taken from a shared free list, and read() waiting for the
+        event, returning the word and giving the pair back.  The product stays
+        ordered on the current stream, as torch's own results are."""
         rt = _hip._rt()
         with _early_lock:
             free = _early_free.setdefault(self.dev.index, [])
@@ -253,6 +256,8 @@ class _TorchFamily:
 
 class _HipFamily:
     """NumPy inputs: device arrays of the HIP runtime on the null stream."""
+
+    stream_ordered = False
 
     def __init__(self):
         if _hip.device_count() < 1:

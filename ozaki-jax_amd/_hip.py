@@ -46,7 +46,6 @@ class _Runtime:
         vp, sz, i = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int
         for name, args in [("hipMalloc", [ctypes.POINTER(vp), sz]), ("hipFree", [vp]),
                            ("hipMemcpy", [vp, vp, sz, i]),
-                           ("hipMemcpyAsync", [vp, vp, sz, i, vp]),
                            ("hipMemset", [vp, i, sz]),
                            ("hipHostFree", [vp]),
                            ("hipStreamDestroy", [vp]),
@@ -113,9 +112,6 @@ class _Runtime:
 
     def host_free(self, p):
         self.check(self.h.hipHostFree(p), "hipHostFree")
-
-    def copy_async(self, dst, src, nbytes, kind):
-        self.check(self.h.hipMemcpyAsync(dst, src, nbytes, kind, None), "hipMemcpyAsync")
 
     def event(self):
         e = ctypes.c_void_p()

@@ -100,7 +100,7 @@ def ozaki_residual_device(fam, At, xt, bt, n_hi, n_lo):
             ws.data_ptr(), wsb, flags.data_ptr(), fam.stream()))
         return fam.read_flags(flags)
 
-    if fused and getattr(fam, "early_flags", None) is not None:
+    if fused and fam.stream_ordered:
         # The fused row kernels (no workspace) have no bounded waits, so the
         # word can hold no OZK_FLAG_WAIT_TIMEOUT, and NaN / Inf are left to
         # propagate as in the reference: a torch result is returned ordered
