@@ -338,23 +338,26 @@ int ozk_wait_flag_word(const uint32_t* host_word, void* stream, uint32_t* flags)
  * word per 512 KiB of it; zero_counts: as many device words, zero before and
  * after.
  * ozk_copy_slots uses `slots` slots of slot_bytes (a multiple of 512 KiB) from
- * slot `first` on, with a HIP event and an owner each (null at first: the
- * stream that used it last), and queues a copy per slot.  To the
- * device (down = 0) it returns when the host array has been read and the
- * copies are queued, to the host when the array is complete.  It waits for a
+ * slot `first` on, with a HIP event each, and queues a copy per slot once the
+ * work queued on `stream` has ended.  To the device it returns when the host
+ * array has been read and the copies are queued, to the host when the array is
+ * complete.  OZK_COPY_UP_NEXT: to the device, without the wait, where nothing
+ * but such copies of the caller's has been queued since one that waited.  It waits for a
  * slot's event before it uses the slot, so calls may follow one another at
  * once.
  * Calls of several threads may share pinned memory, and none waits for what
- * another has queued on its stream: one that finds the memory held, or a slot
- * still queued on another stream, copies without it.  Both return OZK_ERR_HIP on a
+ * another has queued on its stream: ozk_copy_slots take turns, and an
+ * ozk_copy_to_host that finds the memory in use copies without it.  Both return OZK_ERR_HIP on a
  * stream that is being captured, with nothing recorded. */
+#define OZK_COPY_UP 0
+#define OZK_COPY_DOWN 1
+#define OZK_COPY_UP_NEXT 2
 int ozk_copy_to_host(void* host, const void* dev, size_t bytes, void* staging,
                      size_t staging_bytes, uint32_t* flags,
                      uint32_t* zero_counts, int threads, void* stream);
-int ozk_copy_slots(int down, void* dev, void* host, size_t bytes, void* staging,
+int ozk_copy_slots(int way, void* dev, void* host, size_t bytes, void* staging,
                    size_t slot_bytes, int slots, int first,
-                   void* const* events, void** owners, int threads,
-                   void* stream);
+                   void* const* events, int threads, void* stream);
 
 /* ozk_matmul without a workspace argument, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,

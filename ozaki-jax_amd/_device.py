@@ -43,14 +43,16 @@ _NO_GPU = ("ozaki_jax_amd needs a ROCm GPU; there is no CPU implementation "
            "(no HIP device found).")
 
 
-def _numpy_to_torch(a, dev):
+def _numpy_to_torch(a, dev, following=False):
     """A contiguous NumPy array as a device tensor.  Large ones go through
-    the pinned ring (_hip) on torch's current stream."""
+    the pinned ring (_hip) on torch's current stream (following: as
+    _Stager.to_device)."""
     if a.nbytes < _hip._COPY_MIN:
         return torch.from_numpy(a).to(dev)
     t = torch.empty(a.shape, dtype=_TORCH_DTYPES[a.dtype], device=dev)
     with torch.cuda.device(dev):
-        _hip._stager().to_device(t.data_ptr(), a, torch.cuda.current_stream(dev).cuda_stream)
+        _hip._stager().to_device(t.data_ptr(), a, torch.cuda.current_stream(dev).cuda_stream,
+                                 following)
     return t
 
 
@@ -64,6 +66,16 @@ def _torch_to_numpy(t):
     with torch.cuda.device(t.device):
         _hip._stager().to_host(out, t.data_ptr(),
                                torch.cuda.current_stream(t.device).cuda_stream)
+    return out
+
+
+def f64s(fam, *xs):
+    """fam.f64 of each: a staged upload behind another one does not wait for
+    it, so that its host copy overlaps the other's transfer."""
+    out, staged = [], False
+    for x in xs:
+        out.append(fam.f64(x, staged))
+        staged = not is_torch(x) and 8 * out[-1].numel() >= _hip._COPY_MIN
     return out
 
 
@@ -166,7 +178,7 @@ class _TorchFamily:
     def stream(self):
         return torch.cuda.current_stream().cuda_stream
 
-    def f64(self, x):
+    def f64(self, x, following=False):
         """float64 device tensor with contiguous rows holding x's values;
         never aliases a NumPy input."""
         if is_torch(x):
@@ -177,7 +189,7 @@ class _TorchFamily:
                 t = t.to(self.dev)
         else:
             a = np.ascontiguousarray(np.asarray(x, dtype=np.float64))
-            t = _numpy_to_torch(a, self.dev)
+            t = _numpy_to_torch(a, self.dev, following)
         if t.dim() >= 1 and t.numel() > 0 and t.stride(-1) != 1:
             t = t.contiguous()
         if t.dim() == 2 and t.numel() > 0 and t.stride(0) < max(t.shape[1], 1):
@@ -266,10 +278,10 @@ class _HipFamily:
     def stream(self):
         return None
 
-    def f64(self, x):
+    def f64(self, x, following=False):
         if is_torch(x):  # matmul_numpy takes any array-like
             x = x.detach().cpu().numpy()
-        return _hip.DeviceArray.from_numpy(np.asarray(x, dtype=np.float64))
+        return _hip.DeviceArray.from_numpy(np.asarray(x, dtype=np.float64), following)
 
     def empty(self, shape, dtype=np.float64):
         return _hip.DeviceArray(shape, dtype)

@@ -28,6 +28,7 @@ from . import _lib
 
 _ROCM_LIB = "/opt/rocm/lib"
 _H2D, _D2H, _D2D = 1, 2, 3
+_COPY_UP, _COPY_DOWN, _COPY_UP_NEXT = 0, 1, 2  # ozk_copy_slots
 _OP_N, _OP_T = 111, 112  # rocblas_operation_none / _transpose
 
 
@@ -148,24 +149,22 @@ _STAGE_CHUNK = 64 << 20
 
 
 class _Slots:
-    """Pinned slots with an event each (ozk_copy_slots, which sees to it that
-    transfers of several threads do not meet).  The lock hands out the slot a
-    transfer starts at."""
+    """Pinned slots with an event each (ozk_copy_slots).  The lock hands out
+    the slot a transfer starts at."""
 
     def __init__(self, rt, slot, slots):
         self.slot, self.slots, self.first = int(slot), int(slots), 0
         self.buf = rt.host_malloc(self.slot * self.slots)
         self.ev = (ctypes.c_void_p * self.slots)(*[rt.event() for _ in range(self.slots)])
-        self.owners = (ctypes.c_void_p * self.slots)()
         self.lock = threading.Lock()
 
-    def copy(self, down, dev_ptr, host, threads, stream):
+    def copy(self, way, dev_ptr, host, threads, stream):
         with self.lock:
             first = self.first
             self.first = (first + -(-host.nbytes // self.slot)) % self.slots
         _lib.check(_lib.load().ozk_copy_slots(
-            down, dev_ptr, host.ctypes.data, host.nbytes, self.buf, self.slot, self.slots,
-            first, self.ev, self.owners, threads, stream))
+            way, dev_ptr, host.ctypes.data, host.nbytes, self.buf, self.slot, self.slots,
+            first, self.ev, threads, stream))
 
     def release(self, h):
         h.hipHostFree(self.buf)
@@ -177,8 +176,8 @@ class _Stager:
     """Pinned memory of the library's staged copies, allocated once per device
     and kept for the process: slots for the way up, as much memory with a
     flag word and a device counter per 512 KiB for the way down
-    (ozk_copy_to_host), and larger slots for large transfers either way.  A
-    transfer that finds its memory in use by another thread's goes without."""
+    (ozk_copy_to_host), and larger slots for large transfers either way.  The
+    library sees to it that transfers of several threads do not meet."""
 
     def __init__(self, rt, slot=_SLOT, slots=_SLOTS):
         self.rt, self.size = rt, int(slot) * int(slots)
@@ -203,17 +202,20 @@ class _Stager:
                 self.big = _Slots(self.rt, _BIG_SLOT, _BIG_SLOTS)
             return self.big
 
-    def to_device(self, dev_ptr, host, stream=None):
+    def to_device(self, dev_ptr, host, stream=None, following=False):
         """host: a C-contiguous array, whose bytes go to dev_ptr on `stream`.
-        They have been read when this returns; the copy may still run."""
+        They have been read when this returns; the copy may still run.
+        following: nothing but uploads has been queued there since one that
+        waited for the stream."""
         slots = self.up if host.nbytes <= _SLOT * _SLOTS else self._big()
-        slots.copy(0, dev_ptr, host, self._threads(host.nbytes), stream)
+        slots.copy(_COPY_UP_NEXT if following else _COPY_UP, dev_ptr, host,
+                   self._threads(host.nbytes), stream)
 
     def to_host(self, out, dev_ptr, stream=None):
         """out: a C-contiguous array, filled from dev_ptr behind the work
         queued on `stream`."""
         if out.nbytes > _SLOT * _SLOTS:
-            self._big().copy(1, dev_ptr, out, self._threads(out.nbytes), stream)
+            self._big().copy(_COPY_DOWN, dev_ptr, out, self._threads(out.nbytes), stream)
             return
         _lib.check(_lib.load().ozk_copy_to_host(
             out.ctypes.data, dev_ptr, out.nbytes, self.down, self.size, self.flags,
@@ -327,12 +329,13 @@ class DeviceArray:
         return DeviceArray((self.shape[0],), self.dtype, None, self._block, self._offset)
 
     @classmethod
-    def from_numpy(cls, a):
+    def from_numpy(cls, a, following=False):
+        """following: as _Stager.to_device."""
         a = np.ascontiguousarray(a)
         d = cls(a.shape, a.dtype)
         assert d.nbytes == a.nbytes
         if a.nbytes >= _COPY_MIN:
-            _stager().to_device(d.data_ptr(), a)
+            _stager().to_device(d.data_ptr(), a, following=following)
         else:
             _rt().copy(d.data_ptr(), a.ctypes.data, a.nbytes, _H2D)
         return d

@@ -124,7 +124,7 @@ SIGNATURES = {
     "ozk_copy_to_host": (_c_int, [_c_vp, _c_vp, _c_size, _c_vp, _c_size, _c_vp, _c_vp,
                                   _c_int, _c_vp]),
     "ozk_copy_slots": (_c_int, [_c_int, _c_vp, _c_vp, _c_size, _c_vp, _c_size, _c_int, _c_int,
-                                ctypes.POINTER(_c_vp), ctypes.POINTER(_c_vp), _c_int, _c_vp]),
+                                ctypes.POINTER(_c_vp), _c_int, _c_vp]),
     "ozk_matmul_noalloc": (_c_int, [_c_vp, _c_i64, _c_vp, _c_i64, _c_vp, _c_i64, _c_i64,
                                     _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_int,
                                     _c_vp, _c_vp]),

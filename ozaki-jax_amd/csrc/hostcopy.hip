@@ -11,12 +11,15 @@
 // transfers go so both ways, in larger slots, since queued copies also run
 // beside a kernel that holds every CU (a product in row halves).
 //
-// Pinned memory serves one copy at a time, which may hold it while its stream is
-// busy before it.  So that no caller waits for what another has queued, one that
-// finds the memory held, or a slot still queued on another stream, takes the
-// runtime's own copy.  (Waiting for one's stream before taking the memory would
-// do as well, and let all be staged, but cost each copy about 40 us: down 56 ->
-// 95 at 1 MiB, 235 -> 330 at 8.)
+// Pinned memory serves one copy at a time, and no caller waits for what another
+// has queued on its stream.  Copies through slots take turns, each once its
+// stream has drained: queued behind kernels they would keep the slots, and the
+// DMA engine they are queued on, from everyone.  (The second of two uploads in a
+// row goes behind the first all the same: a product of 400^3 NumPy arrays takes
+// 235 us, 265 where it waits.)  The small copy down, a kernel, does not
+// wait either, which would cost it about 40 us (56 -> 95 at 1 MiB, 235 -> 330 at
+// 8): it holds the memory from its launch on, and a caller that finds it held
+// takes the runtime's own copy.
 #include <atomic>
 #include <condition_variable>
 #include <mutex>
@@ -31,19 +34,12 @@ namespace ozk {
 constexpr size_t kPiece = 512 << 10;
 constexpr uintptr_t kHugePage = 2 << 20;
 
-// Held while a copy uses the pinned memory at `staging`; no one waits for it.
-// (Other memory may share the mutex: a copy then goes without.)
-static std::mutex& staging_turn(const void* staging) {
-  static std::mutex turns[64];
-  return turns[((uintptr_t)staging >> 20) % 64];
-}
-
-// The runtime's own copy, in its place.
-static int copy_direct(bool down, void* dev, void* host, size_t bytes, hipStream_t st) {
-  OZK_HIP(hipMemcpyAsync(down ? host : dev, down ? dev : host, bytes,
-                         down ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, st));
-  OZK_HIP(hipStreamSynchronize(st));
-  return OZK_OK;
+// Held while a copy uses the pinned memory at `staging`, of copy_out or of
+// copy_slots.  (Other memory of the same kind may share the mutex; of the other
+// kind not, since copy_out holds it while its stream is busy.)
+static std::mutex& staging_turn(const void* staging, bool slots) {
+  static std::mutex turns[2][64];
+  return turns[slots][((uintptr_t)staging >> 20) % 64];
 }
 
 // ---------------------------------------------------------------- down
@@ -247,8 +243,12 @@ static void run_threads(Job& job, int threads) {
 static int copy_out(void* host, const void* dev, size_t bytes, void* staging,
                     size_t staging_bytes, uint32_t* flags, uint32_t* count, int threads,
                     hipStream_t st) {
-  const std::unique_lock<std::mutex> turn(staging_turn(staging), std::try_to_lock);
-  if (!turn.owns_lock()) return copy_direct(true, (void*)dev, host, bytes, st);
+  const std::unique_lock<std::mutex> turn(staging_turn(staging, false), std::try_to_lock);
+  if (!turn.owns_lock()) {
+    OZK_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
+    OZK_HIP(hipStreamSynchronize(st));
+    return OZK_OK;
+  }
   const size_t half = staging_bytes / 2;
   const bool one = bytes <= staging_bytes;
   OutJob job(one ? 1 : (bytes + half - 1) / half);
@@ -268,6 +268,9 @@ static int copy_out(void* host, const void* dev, size_t bytes, void* staging,
                       std::memory_order_relaxed);
   }
   for (size_t b = 0; b < job.batches() && b < 2; ++b) job.launch(b);
+  // (has the runtime queue a completion signal now, while the copy runs: the
+  // next upload's look at the stream would have to wait for one)
+  (void)hipStreamQuery(st);
   const size_t pieces = (bytes + kPiece - 1) / kPiece;
   run_threads(job, (size_t)threads < pieces ? threads : (int)pieces);
   if (job.failed()) {
@@ -354,20 +357,15 @@ struct SlotJob {
   }
 };
 
-static int copy_slots(bool down, void* dev, void* host, size_t bytes, void* staging,
-                      size_t slot_bytes, int slots, int first, void* const* events,
-                      void** owners, int threads, hipStream_t st) {
-  const std::unique_lock<std::mutex> turn(staging_turn(staging), std::try_to_lock);
-  if (!turn.owns_lock()) return copy_direct(down, dev, host, bytes, st);
+static int copy_slots(int way, void* dev, void* host, size_t bytes, void* staging,
+                      size_t slot_bytes, int slots, int first, void* const* events, int threads,
+                      hipStream_t st) {
+  // (asked first: an idle null stream takes 40 us to synchronise)
+  if (way != OZK_COPY_UP_NEXT && hipStreamQuery(st) != hipSuccess)
+    OZK_HIP(hipStreamSynchronize(st));
+  const std::lock_guard<std::mutex> turn(staging_turn(staging, true));
   SlotJob job((bytes + slot_bytes - 1) / slot_bytes);
-  const int used = job.chunks() < (size_t)slots ? (int)job.chunks() : slots;
-  for (int c = 0; c < used; ++c) {
-    const int k = (first + c) % slots;
-    if (owners[k] != st && hipEventQuery((hipEvent_t)events[k]) == hipErrorNotReady)
-      return copy_direct(down, dev, host, bytes, st);
-  }
-  for (int c = 0; c < used; ++c) owners[(first + c) % slots] = st;
-  job.down = down;
+  job.down = way == OZK_COPY_DOWN;
   job.host = (char*)host;
   job.dev = (char*)dev;
   job.bytes = bytes;
@@ -383,7 +381,7 @@ static int copy_slots(bool down, void* dev, void* host, size_t bytes, void* stag
     job.left[c].store((int)((job.chunk_bytes(c) + kPiece - 1) / kPiece),
                       std::memory_order_relaxed);
   }
-  for (size_t c = 0; down && c < job.chunks() && c < (size_t)slots; ++c) {
+  for (size_t c = 0; job.down && c < job.chunks() && c < (size_t)slots; ++c) {
     job.ok(hipEventSynchronize(job.event(c)));  // an earlier call's copy
     job.issue(c);
   }
@@ -432,20 +430,21 @@ int ozk_copy_to_host(void* host, const void* dev, size_t bytes, void* staging,
   }
 }
 
-int ozk_copy_slots(int down, void* dev, void* host, size_t bytes, void* staging,
-                   size_t slot_bytes, int slots, int first, void* const* events,
-                   void** owners, int threads, void* stream) {
+int ozk_copy_slots(int way, void* dev, void* host, size_t bytes, void* staging,
+                   size_t slot_bytes, int slots, int first, void* const* events, int threads,
+                   void* stream) {
   clear_error();
+  OZK_CHECK_ARG(way >= OZK_COPY_UP && way <= OZK_COPY_UP_NEXT, "staged copy: way %d", way);
   OZK_CHECK_ARG(slots >= 1 && first >= 0 && threads >= 1 && slot_bytes >= kPiece &&
                     slot_bytes % kPiece == 0,
                 "staged copy: invalid ring (%d slots of %zu bytes)", slots, slot_bytes);
   if (bytes == 0) return OZK_OK;
-  OZK_CHECK_ARG(host && dev && staging && events && owners, "null pointer");
+  OZK_CHECK_ARG(host && dev && staging && events, "null pointer");
   const int rc = refuse_capture((hipStream_t)stream);
   if (rc) return rc;
   try {
-    return copy_slots(down != 0, dev, host, bytes, staging, slot_bytes, slots, first, events,
-                      owners, threads, (hipStream_t)stream);
+    return copy_slots(way, dev, host, bytes, staging, slot_bytes, slots, first, events,
+                      threads, (hipStream_t)stream);
   } catch (const std::exception& e) {
     set_error("staged copy: %s", e.what());
     return OZK_ERR_HIP;
