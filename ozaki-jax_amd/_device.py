@@ -72,10 +72,9 @@ def _torch_to_numpy(t):
 def f64s(fam, *xs):
     """fam.f64 of each: a staged upload behind another one does not wait for
     it, so that its host copy overlaps the other's transfer."""
-    out, staged = [], False
-    for x in xs:
-        out.append(fam.f64(x, staged))
-        staged = not is_torch(x) and 8 * out[-1].numel() >= _hip._COPY_MIN
+    out = [fam.f64(xs[0])]
+    for before, x in zip(xs, xs[1:]):
+        out.append(fam.f64(x, out[-1].nbytes >= _hip._COPY_MIN and not is_torch(before)))
     return out
 
 

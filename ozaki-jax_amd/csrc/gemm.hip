@@ -1627,39 +1627,52 @@ size_t gemm_state_bytes(int64_t N, int64_t M, int pipe, int nhi, int nlo, int or
 //
 // P is the one that minimises nst / P + split_cost(), both in stages of one
 // tile: the sums written and read again (200 KB RB per piece for 24 pairs), the
-// fixup's launch and its walk over the P pieces of a tile.  The pairs of the
-// schedule do not enter, since the stage and the sums both grow with them.
+// fixup's launch and its walk over the P pieces of a tile.  Both the stage and
+// the sums grow with the pairs of the schedule, the sums faster, since a stage
+// has a part that does not (stage_us): with few pairs a split costs fewer stages.
 // Pieces of kMinPieceStages or more keep the workspace no larger than that of
 // P = min(cus / T, nst / kMinPieceStages) on the usual tiles.
-// Fitted to the whole call at 24 pairs (us; without a split / the P it picks / that P):
+// Over 160 shapes (3, 8, 12, 15 and 24 pairs, RB 1 to 3, T 1 to 242, nst 32 to
+// 375) the call takes 0.4% more on average than with the best P and tiles, and
+// 9% with that P on the usual tiles.
+// The whole call at 24 pairs (us; without a split / the P it picks / that P):
 //   RB 1, nst 64:  T 2 55 / 38 / 38,  T 64 58 / 53 / 54,  T 128 60 / 60 / 68
 //   RB 1, nst 32:  T 2 33 / 33 / 34,  T 32 37 / 37 / 43,  T 128 42 / 42 / 55
 //   RB 1, nst 128: T 8 98 / 47 / 47,  T 32 97 / 55 / 56,  T 128 102 / 91 / 91
 //   RB 2, nst 64:  T 16 152 / 137 / 137,  T 64 153 / 153 / 173
 //   RB 2, nst 128: T 16 281 / 222 / 224,  T 64 283 / 259 / 275
+// and at 3 and 8 pairs, RB 3, nst 128, T 128 behind a whole round: 150 / 136 /
+// 136 and 203 / 196 / 196.
 constexpr int kMinPieceStages = 16;
 
-static double split_cost(int64_t T, int64_t P, int rb) {
-  return (rb == 1 ? 1.0 : 1.6) * (15.0 + (double)P + (double)(T * P) / 10);
+static double split_cost(int64_t T, int64_t P, int np, int rb) {
+  const double unit = rb == 1 ? 1.0 : np < 14 ? 1.2 + 0.03 * np : 1.6;
+  return unit * (15.0 + (double)P + (double)(T * P) / 10);
 }
+
+// A stage, in microseconds: fitted to the same calls, within 10%.
+static double stage_us(int np, int rb) { return 0.45 + 0.0075 * np * rb; }
 
 struct TailPlan {
   int P = 0;        // pieces per tail tile (0: no split)
   int64_t T = 0;    // tail tiles
   int grid = 0;     // all-pairs workgroups
   size_t bytes = 0; // partial sums
+  double stages = 0;  // time of the launch by the model
 };
 
 static TailPlan plan_tail(int64_t ntiles, int cus, int64_t nst, int np, int rb) {
   TailPlan tp;
   const int64_t R = ntiles / cus, T = ntiles % cus;
+  tp.stages = (double)(R * nst);
   if (T == 0) return tp;
   int64_t P = 1;
   double best = (double)nst;
   for (int64_t p = 2; p <= cus / T && p <= nst / kMinPieceStages; ++p) {
-    const double c = (double)nst / (double)p + split_cost(T, p, rb);
+    const double c = (double)nst / (double)p + split_cost(T, p, np, rb);
     if (c < best) best = c, P = p;
   }
+  tp.stages += best;
   if (P < 2) return tp;
   tp.P = (int)P;
   tp.T = T;
@@ -1698,13 +1711,26 @@ static int allpairs_tm(int pipe, int nhi, int nlo, bool sym) {
                                      : ap_rb(nhi, nlo, 0, 2, sym));
 }
 
-// Whether an N x M product takes the 32-row tiles: if all of them fit the CUs
-// at once.  (A second round would cost more than the larger tiles: a stage
-// takes 0.6 us at 32 rows and 0.96 at 64 for 24 pairs, since a stage of 32 rows
-// is bound by LDS, 110 KB a stage, and no longer by its MFMAs.)
-static bool use_small(int64_t N, int64_t M, int pipe, int nhi, int nlo, int order, bool sym) {
-  return !sym && small_form(pipe, nhi, nlo, order) &&
-         allpairs_ntiles(N, M, false, kSmallTM) <= cu_count();
+// Whether an N x M product of nst stages takes the 32-row tiles: if all of them
+// fit the CUs at once, unless K is so long that the usual tiles, fewer and so
+// in more pieces, are faster by the model (by 12%: it is that exact).  A second
+// round would cost more than the larger tiles: a stage takes 0.64 us at 32 rows
+// and 0.77 at 64 for 24 pairs, since its barrier and the wait for its loads
+// do not shrink (matrix cores busy 31% of the launch at 512 x 4096 x 512, 63% with
+// 64-row tiles at 1024 x 4096 x 1024; LDS 13% and 20%).  Long K, 32-row tiles ->
+// the usual (us): 24 pairs 384 x 24000 x 512 278 -> 260, 700 x 24000 x 700 445 ->
+// 433; at 384 x 12000 x 512 they would take 167 (156).  tail_bytes: what there
+// is for the pieces' sums.
+static bool use_small(int64_t N, int64_t M, int64_t nst, int pipe, int nhi, int nlo, int order,
+                      bool sym, size_t tail_bytes) {
+  const int cus = cu_count();
+  const int64_t ntiles = allpairs_ntiles(N, M, false, kSmallTM);
+  if (sym || !small_form(pipe, nhi, nlo, order) || ntiles > cus) return false;
+  if (allpairs_sweeps(pipe, nhi, nlo) != 1) return true;
+  const int np = pair_count(pipe, nhi, nlo), tm = allpairs_tm(pipe, nhi, nlo, false);
+  const double small = stage_us(np, 1) * plan_tail(ntiles, cus, nst, np, 1).stages;
+  const TailPlan usual = plan_tail(allpairs_ntiles(N, M, false, tm), cus, nst, np, tm / 32);
+  return usual.bytes > tail_bytes || stage_us(np, tm / 32) * usual.stages >= 0.88 * small;
 }
 
 static int64_t allpairs_nst(int64_t K, bool i8) {
@@ -1717,7 +1743,8 @@ static int64_t allpairs_nst(int64_t K, bool i8) {
 size_t gemm_tail_bytes(int64_t N, int64_t M, int64_t K, int pipe, int nhi, int nlo,
                        bool sym, bool i8) {
   if (!allpairs_schedule(pipe, nhi, nlo) || allpairs_sweeps(pipe, nhi, nlo) != 1) return 0;
-  const int tm = use_small(N, M, pipe, nhi, nlo, OZK_ORDER_2SUM, sym)
+  const int tm = use_small(N, M, allpairs_nst(K, i8), pipe, nhi, nlo, OZK_ORDER_2SUM, sym,
+                           SIZE_MAX)
                      ? kSmallTM
                      : allpairs_tm(pipe, nhi, nlo, sym);
   return plan_tail(allpairs_ntiles(N, M, sym, tm), cu_count(), allpairs_nst(K, i8),
@@ -1748,7 +1775,11 @@ static int launch_allpairs(bool i8, int pipe, const void* As, const int32_t* Ae,
   }
   ApArgs a;
   const int64_t al = round_up(N, kLinePad), bl = round_up(M, kLinePad);
-  a.small = use_small(N, M, pipe, nhi, nlo, order, sym);
+  // workspace: fold state | dynamic-tail words | K-split partial sums
+  const size_t off = round_up((int64_t)need, 256);
+  const size_t tail_off = off + kDynBytes;
+  a.small = use_small(N, M, allpairs_nst(K, i8), pipe, nhi, nlo, order, sym,
+                      state && state_bytes > tail_off ? state_bytes - tail_off : 0);
   const int tmr = a.small ? kSmallTM : allpairs_tm(pipe, nhi, nlo, sym);
   const int64_t ntiles = allpairs_ntiles(N, M, sym, tmr);
   OZK_CHECK_ARG(ntiles < (1ll << 31), "problem too large for one launch");
@@ -1761,17 +1792,15 @@ static int launch_allpairs(bool i8, int pipe, const void* As, const int32_t* Ae,
   a.part = nullptr;
   a.dyn = nullptr;
   a.cus = cus;
-  // workspace: fold state | dynamic-tail words | K-split partial sums
-  const size_t off = round_up((int64_t)need, 256);
   if (allpairs_sweeps(pipe, nhi, nlo) == 1) {
     const TailPlan tp = plan_tail(ntiles, cus, allpairs_nst(K, i8),
                                   pair_count(pipe, nhi, nlo), tmr / 32);
-    if (tp.P > 1 && state && state_bytes >= off + kDynBytes + tp.bytes) {
+    if (tp.P > 1 && state && state_bytes >= tail_off + tp.bytes) {
       a.grid = dim3((unsigned)tp.grid);
       a.tail_P = tp.P;
       a.tail_T = tp.T;
       a.tile0 = (int)(ntiles - tp.T);
-      a.part = (uint32_t*)((char*)state + off + kDynBytes);
+      a.part = (uint32_t*)((char*)state + tail_off);
     }
   }
   // the dynamic tail's counters, when some sweep will use them (each sweep

@@ -19,13 +19,17 @@ def operands(N, K, M):
 # One row or column; both sides of 32 and 64 rows; 256 tiles of 32 rows (the
 # last shape that takes them) and more; one stage and a ragged last one.  With K
 # split: 4 tiles on BF16 and INT8 planes, 256 tiles in 2 pieces, 16 tiles
-# after a round of 64-row ones, and (medium) of 96-row ones.
+# after a round of 64-row ones, and (medium) of 96-row ones.  Long K, where the
+# usual tiles come back (64 and 96 rows), and where they do not yet.  128 tiles
+# of 96 rows after a round, of the fewest pairs.
 @pytest.mark.parametrize("shape,precision", [
     ((1, 1, 1), "high"), ((31, 33, 64), "high"), ((33, 32, 65), "max"), ((65, 300, 63), "medium"),
     ((1024, 70, 512), "high"), ((1024, 70, 512), "max"), ((1024, 70, 512), "medium"),
     ((1025, 70, 512), "high"), ((1025, 70, 512), "medium"),
     ((40, 4096, 60), "high"), ((40, 8200, 60), "high"), ((40, 8200, 60), "medium"),
-    ((500, 4090, 510), "high"), ((1056, 4200, 1024), "high"), ((1600, 4200, 1030), "medium")])
+    ((500, 4090, 510), "high"), ((1056, 4200, 1024), "high"), ((1600, 4200, 1030), "medium"),
+    ((384, 24000, 512), "high"), ((384, 24000, 512), "medium"), ((384, 12000, 512), "high"),
+    ((1536, 4096, 1536), (1, 1))])
 def test_few_tiles_ondevice(ozk, shape, precision):
     N, K, M = shape
     A, B = operands(N, K, M)
