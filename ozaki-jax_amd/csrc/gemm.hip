@@ -796,8 +796,16 @@ __global__ __launch_bounds__(kThreads16) void gemm_allpairs(
   // (a wave that issues no stage loads; the symmetric form, whose scalar
   // registers are short, ran 1.2% slower with this and takes
   // publish_flags_kernel)
-  if constexpr (!SYM)
+  // (The loop behind it is allocated differently for the two ways to write the
+  // test.  Schedules (2, 1) and (2, 2) take the second: 3001 x 24000 x 1300 in
+  // 1100 and 1345 us against 1129 and 1356, 1100 and 1344 before flags were
+  // published here; (1, 1) 853 against 827, (4, 1) the same.)
+  if constexpr (!SYM && PIPE == OZK_PIPE_ONDEVICE && NHI == 2 && NLO <= 2) {
+    if (__builtin_expect(bid == 0, 0))
+      if (threadIdx.x == 256 && pub.host) publish_flags(pub);
+  } else if constexpr (!SYM) {
     if (pub.host && bid == 0 && threadIdx.x == 256) publish_flags(pub);
+  }
   // SYM: B's planes are A's (a gram matrix); only tiles tm <= tn are run
   // and each element folds both C[i][j] and C[j][i] (see the epilogue).
   static_assert(!SYM || (B0 == 0 && B1 == 2 && ORDER == OZK_ORDER_2SUM),
