@@ -43,16 +43,16 @@ _NO_GPU = ("ozaki_jax_amd needs a ROCm GPU; there is no CPU implementation "
            "(no HIP device found).")
 
 
-def _numpy_to_torch(a, dev, following=False):
+def _numpy_to_torch(a, dev, place=_hip.ALONE):
     """A contiguous NumPy array as a device tensor.  Large ones go through
-    the pinned ring (_hip) on torch's current stream (following: as
-    _Stager.to_device)."""
-    if a.nbytes < _hip._COPY_MIN:
+    the pinned slots (_hip) on torch's current stream (place: as
+    DeviceArray.from_numpy)."""
+    if a.nbytes < (_hip._ALONE_MIN if place == _hip.ALONE else _hip._COPY_MIN):
         return torch.from_numpy(a).to(dev)
     t = torch.empty(a.shape, dtype=_TORCH_DTYPES[a.dtype], device=dev)
     with torch.cuda.device(dev):
         _hip._stager().to_device(t.data_ptr(), a, torch.cuda.current_stream(dev).cuda_stream,
-                                 following)
+                                 place == _hip.FOLLOWING)
     return t
 
 
@@ -72,9 +72,16 @@ def _torch_to_numpy(t):
 def f64s(fam, *xs):
     """fam.f64 of each: a staged upload behind another one does not wait for
     it, so that its host copy overlaps the other's transfer."""
-    out = [fam.f64(xs[0])]
-    for before, x in zip(xs, xs[1:]):
-        out.append(fam.f64(x, out[-1].nbytes >= _hip._COPY_MIN and not is_torch(before)))
+    large = [isinstance(x, np.ndarray) and 8 * x.size >= _hip._COPY_MIN for x in xs]
+    place = _hip.FIRST if sum(large) > 1 else _hip.ALONE
+    out = []
+    for x, staged in zip(xs, large):
+        out.append(fam.f64(x, place))
+        if place != _hip.ALONE:
+            if staged:
+                place = _hip.FOLLOWING
+            elif is_torch(x):  # may have queued a conversion
+                place = _hip.FIRST
     return out
 
 
@@ -177,7 +184,7 @@ class _TorchFamily:
     def stream(self):
         return torch.cuda.current_stream().cuda_stream
 
-    def f64(self, x, following=False):
+    def f64(self, x, place=_hip.ALONE):
         """float64 device tensor with contiguous rows holding x's values;
         never aliases a NumPy input."""
         if is_torch(x):
@@ -188,7 +195,7 @@ class _TorchFamily:
                 t = t.to(self.dev)
         else:
             a = np.ascontiguousarray(np.asarray(x, dtype=np.float64))
-            t = _numpy_to_torch(a, self.dev, following)
+            t = _numpy_to_torch(a, self.dev, place)
         if t.dim() >= 1 and t.numel() > 0 and t.stride(-1) != 1:
             t = t.contiguous()
         if t.dim() == 2 and t.numel() > 0 and t.stride(0) < max(t.shape[1], 1):
@@ -277,10 +284,10 @@ class _HipFamily:
     def stream(self):
         return None
 
-    def f64(self, x, following=False):
+    def f64(self, x, place=_hip.ALONE):
         if is_torch(x):  # matmul_numpy takes any array-like
             x = x.detach().cpu().numpy()
-        return _hip.DeviceArray.from_numpy(np.asarray(x, dtype=np.float64), following)
+        return _hip.DeviceArray.from_numpy(np.asarray(x, dtype=np.float64), place)
 
     def empty(self, shape, dtype=np.float64):
         return _hip.DeviceArray(shape, dtype)

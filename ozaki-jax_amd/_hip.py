@@ -138,10 +138,14 @@ class _Runtime:
 
 
 # Host copies of at least _COPY_MIN bytes go through pinned memory
-# (_Stager); smaller ones are as fast as the runtime's own copies.  Those above
-# _SLOTS * _SLOT bytes take the larger slots.  Products whose halves reach _STAGE_MIN bytes
-# run in two halves (matmul).
+# (_Stager); smaller ones are as fast as the runtime's own copies.  So is an
+# upload below _ALONE_MIN that no other follows or precedes (1, 4, 8, 32 MiB: 60,
+# 142, 250, 960 us; staged 75, 165, 265, 880): staging gains from the overlap of
+# two.  Those above _SLOTS * _SLOT bytes take the larger slots.  Products whose
+# halves reach _STAGE_MIN bytes run in two halves (matmul).
 _COPY_MIN = 1 << 20
+_ALONE_MIN = 16 << 20
+ALONE, FIRST, FOLLOWING = 0, 1, 2  # place of an upload among several (from_numpy)
 _SLOTS, _SLOT = 8, 4 << 20
 _BIG_SLOTS, _BIG_SLOT = 4, 32 << 20
 _STAGE_MIN = 32 << 20
@@ -329,13 +333,14 @@ class DeviceArray:
         return DeviceArray((self.shape[0],), self.dtype, None, self._block, self._offset)
 
     @classmethod
-    def from_numpy(cls, a, following=False):
-        """following: as _Stager.to_device."""
+    def from_numpy(cls, a, place=ALONE):
+        """place: FIRST of several uploads, or FOLLOWING others with nothing
+        else queued since the first."""
         a = np.ascontiguousarray(a)
         d = cls(a.shape, a.dtype)
         assert d.nbytes == a.nbytes
-        if a.nbytes >= _COPY_MIN:
-            _stager().to_device(d.data_ptr(), a, following=following)
+        if a.nbytes >= (_ALONE_MIN if place == ALONE else _COPY_MIN):
+            _stager().to_device(d.data_ptr(), a, following=place == FOLLOWING)
         else:
             _rt().copy(d.data_ptr(), a.ctypes.data, a.nbytes, _H2D)
         return d

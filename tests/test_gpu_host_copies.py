@@ -44,14 +44,14 @@ def test_slots_refuse_a_captured_stream(ozk, mode):
 
 
 def test_residual_with_numpy_operands_refuses_capture(ozk):
-    """A fused residual of tensors reads no flags; with b as a NumPy array of
-    1 MiB its upload is what a capture must refuse."""
+    """A fused residual of tensors reads no flags; with b as a NumPy array its
+    staged upload (16 MiB) is what a capture must refuse."""
     import torch
     from ozaki_jax_amd import _lib
     rng = np.random.RandomState(2)
-    A = torch.from_numpy(rng.randn(1 << 17, 8)).cuda()
+    A = torch.from_numpy(rng.randn(1 << 21, 8)).cuda()
     x = torch.from_numpy(rng.randn(8)).cuda()
-    b = rng.randn(1 << 17)
+    b = rng.randn(1 << 21)
     want = ozk.residual(A, x, torch.from_numpy(b).cuda(), mode="ozaki")
     case("residual with a NumPy b under capture")
     g = torch.cuda.CUDAGraph()
@@ -133,3 +133,38 @@ def test_copies_do_not_wait_for_another_threads_stream(ozk, way, mib):
     for i in range(2):
         assert np.array_equal(got[i] if way == "down" else got[i].cpu().numpy(), a[i])
     assert early, "the copy waited for the other thread's stream"
+
+
+@pytest.mark.parametrize("torch_family", [False, True])
+def test_f64s_by_place(ozk, monkeypatch, torch_family):
+    """Which uploads are staged, and which of them follow another without a
+    wait: sizes around the thresholds, alone and in rows."""
+    import torch
+    from ozaki_jax_amd import _device as D, _hip
+    fam = D.family(torch_family)
+    seen = []
+    to_device = _hip._Stager.to_device
+
+    def spy(self, ptr, host, stream=None, following=False):
+        seen.append((host.nbytes, following))
+        return to_device(self, ptr, host, stream, following)
+
+    monkeypatch.setattr(_hip._Stager, "to_device", spy)
+    rng = np.random.RandomState(3)
+    mib = 1 << 17
+    small, one, four, big = (rng.randn(n) for n in (mib - 1, mib, 4 * mib, 16 * mib))
+    tensor = torch.ones(2 * mib, dtype=torch.float32, device="cuda")
+    rows = [([one], []), ([big], [False]), ([four, small], []),
+            ([one, four], [False, True]), ([one, small, four], [False, True]),
+            ([four.astype(np.float32), one, big], [False, True, True])]
+    if torch_family:
+        rows.append(([one, tensor, four, one], [False, False, True]))
+    for xs, want in rows:
+        del seen[:]
+        case(f"f64s of {[x.nbytes if isinstance(x, np.ndarray) else 'tensor' for x in xs]}")
+        out = D.f64s(fam, *xs)
+        assert [f for _, f in seen] == want
+        for x, t in zip(xs, out):
+            got = t.cpu().numpy() if torch_family else t.numpy()
+            x = x if isinstance(x, np.ndarray) else x.cpu().numpy()
+            assert np.array_equal(got, x.astype(np.float64))
