@@ -342,13 +342,14 @@ int ozk_wait_flag_word(const uint32_t* host_word, void* stream, uint32_t* flags)
  * work queued on `stream` has ended.  To the device it returns when the host
  * array has been read and the copies are queued, to the host when the array is
  * complete.  OZK_COPY_UP_NEXT: to the device, without the wait, where nothing
- * but such copies of the caller's has been queued since one that waited.  It waits for a
- * slot's event before it uses the slot, so calls may follow one another at
- * once.
+ * but such copies of the caller's has been queued since one that waited.  It
+ * waits for a slot's event before it uses the slot, so calls may follow one
+ * another at once.
  * Calls of several threads may share pinned memory, and none waits for what
  * another has queued on its stream: ozk_copy_slots take turns, and an
- * ozk_copy_to_host that finds the memory in use copies without it.  Both return OZK_ERR_HIP on a
- * stream that is being captured, with nothing recorded. */
+ * ozk_copy_to_host that finds the memory in use copies without it.  Both
+ * return OZK_ERR_HIP on a stream that is being captured, with nothing
+ * recorded. */
 #define OZK_COPY_UP 0
 #define OZK_COPY_DOWN 1
 #define OZK_COPY_UP_NEXT 2

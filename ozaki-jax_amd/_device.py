@@ -58,7 +58,7 @@ def _numpy_to_torch(a, dev, place=_hip.ALONE):
 
 def _torch_to_numpy(t):
     """A device tensor as a new NumPy array, large contiguous ones through the
-    pinned ring (_hip) on torch's current stream."""
+    pinned memory (_hip) on torch's current stream."""
     if (not t.is_cuda or not t.is_contiguous() or t.dtype not in _NUMPY_DTYPES
             or t.numel() * t.element_size() < _hip._COPY_MIN):
         return t.cpu().numpy()

@@ -522,7 +522,7 @@ def _pool():
 
 
 def _stager():
-    """The current device's ring."""
+    """The current device's pinned memory for host copies."""
     return _get(("stager", _rt().device()), lambda: _Stager(_rt()))
 
 

@@ -13,7 +13,7 @@
 //     diagonal block for its rows c .. c+31 (the U12 block);
 //  3. lu_update_kernel: trailing A22 -= L21 U12, 64 x 64 tiles, K = 32.
 // The panel step is the critical path: 32 pivot searches, one workgroup
-// barrier each (about 0.7 us).
+// barrier each (about 0.9 us).
 #include <cfloat>
 
 #include "common.h"
@@ -63,7 +63,10 @@ __device__ __forceinline__ uint32_t lu_wave_reduce(uint32_t u) {
 //
 // What bounds it: one workgroup on one CU, 32 dependent column steps.  Each
 // step is a chain of a pivot search, an LDS exchange with one barrier and
-// the rank-1 update.  The steps run as a rolled loop: unrolled over the 32
+// the rank-1 update: 0.9 us at one row slot, 28.8 a panel.  What taller panels
+// take beyond that (34.9 us at 2 slots, 42.4 at 4, 51.9 at 6, 76.2 at 8) is the
+// vector work and the loads of one CU, and at 7 and 8 slots, and from 5 on
+// without 16-byte rows, registers spilled to scratch.  The steps run as a rolled loop: unrolled over the 32
 // columns the kernel was 28000 instructions, and fetching that much
 // straight-line code (200 KB, over the 64 KB instruction cache) cost about
 // a sixth of every short step and more of the tall ones.  The loop needs the active column
@@ -71,7 +74,7 @@ __device__ __forceinline__ uint32_t lu_wave_reduce(uint32_t u) {
 // updated columns move down and the finished L entry enters at the end.
 // Measured with the row slots a compile-time count, the loads and stores
 // four lanes a row and the permutation composed in parallel (us a panel,
-// unrolled -> rolled): 4096 rows 108 -> 88, 2048 71 -> 45, 512 46 -> 30; n =
+// unrolled -> rolled): 4096 rows 108 -> 83, 2048 71 -> 45, 512 46 -> 30; n =
 // 4096 factored in 9.1 ms (12.7; 8.7 with the update below).  Four waves (one
 // a SIMD) instead of eight were slower (55 at 2048 rows), reading the pivot row
 // back from LDS instead of by readlane too (50).
