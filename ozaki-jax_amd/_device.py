@@ -73,15 +73,15 @@ def f64s(fam, *xs):
     """fam.f64 of each: a staged upload behind another one does not wait for
     it, so that its host copy overlaps the other's transfer."""
     large = [isinstance(x, np.ndarray) and 8 * x.size >= _hip._COPY_MIN for x in xs]
-    place = _hip.FIRST if sum(large) > 1 else _hip.ALONE
-    out = []
+    if large.count(True) < 2:
+        return [fam.f64(x) for x in xs]
+    place, out = _hip.FIRST, []
     for x, staged in zip(xs, large):
         out.append(fam.f64(x, place))
-        if place != _hip.ALONE:
-            if staged:
-                place = _hip.FOLLOWING
-            elif is_torch(x):  # may have queued a conversion
-                place = _hip.FIRST
+        if staged:
+            place = _hip.FOLLOWING
+        elif is_torch(x):  # may have queued a conversion
+            place = _hip.FIRST
     return out
 
 
@@ -127,9 +127,10 @@ class FlagWords:
         lib = _lib.load()
         self.word.value = 0
         rc = call(self.dev, self.host)
-        if rc < 0 and rc != _lib.OZK_ERR_HIP:  # refused before anything was queued
-            self.give_back()
-        _lib.check(rc)
+        if rc < 0:
+            if rc != _lib.OZK_ERR_HIP:  # refused before anything was queued
+                self.give_back()
+            _lib.check(rc)
         fl = ctypes.c_uint32()
         _lib.check(lib.ozk_wait_flag_word(self.host, stream, ctypes.byref(fl)))
         self.give_back()

@@ -139,12 +139,12 @@ class _Runtime:
 
 # Host copies of at least _COPY_MIN bytes go through pinned memory
 # (_Stager); smaller ones are as fast as the runtime's own copies.  So is an
-# upload below _ALONE_MIN that no other follows or precedes (1, 4, 8, 32 MiB: 60,
-# 142, 250, 960 us; staged 75, 165, 265, 880): staging gains from the overlap of
-# two.  Those above _SLOTS * _SLOT bytes take the larger slots.  Products whose
+# upload below _ALONE_MIN that no other follows or precedes, since staging gains
+# from the overlap of two (host products of an array of 1, 2, 4, 8, 12 MiB with a
+# small one: 177, 211, 321, 535, 715 us; staged 190, 240, 346, 490, 610).  Those above _SLOTS * _SLOT bytes take the larger slots.  Products whose
 # halves reach _STAGE_MIN bytes run in two halves (matmul).
 _COPY_MIN = 1 << 20
-_ALONE_MIN = 16 << 20
+_ALONE_MIN = 6 << 20
 ALONE, FIRST, FOLLOWING = 0, 1, 2  # place of an upload among several (from_numpy)
 _SLOTS, _SLOT = 8, 4 << 20
 _BIG_SLOTS, _BIG_SLOT = 4, 32 << 20
