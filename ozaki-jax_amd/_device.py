@@ -43,16 +43,14 @@ _NO_GPU = ("ozaki_jax_amd needs a ROCm GPU; there is no CPU implementation "
            "(no HIP device found).")
 
 
-def _numpy_to_torch(a, dev, place=_hip.ALONE):
+def _numpy_to_torch(a, dev):
     """A contiguous NumPy array as a device tensor.  Large ones go through
-    the pinned slots (_hip) on torch's current stream (place: as
-    DeviceArray.from_numpy)."""
-    if a.nbytes < (_hip._ALONE_MIN if place == _hip.ALONE else _hip._COPY_MIN):
+    the pinned slots (_hip) on torch's current stream."""
+    if a.nbytes < _hip._ALONE_MIN:
         return torch.from_numpy(a).to(dev)
     t = torch.empty(a.shape, dtype=_TORCH_DTYPES[a.dtype], device=dev)
     with torch.cuda.device(dev):
-        _hip._stager().to_device(t.data_ptr(), a, torch.cuda.current_stream(dev).cuda_stream,
-                                 place == _hip.FOLLOWING)
+        _hip._stager().to_device(t.data_ptr(), a, torch.cuda.current_stream(dev).cuda_stream)
     return t
 
 
@@ -66,22 +64,6 @@ def _torch_to_numpy(t):
     with torch.cuda.device(t.device):
         _hip._stager().to_host(out, t.data_ptr(),
                                torch.cuda.current_stream(t.device).cuda_stream)
-    return out
-
-
-def f64s(fam, *xs):
-    """fam.f64 of each: a staged upload behind another one does not wait for
-    it, so that its host copy overlaps the other's transfer."""
-    large = [isinstance(x, np.ndarray) and 8 * x.size >= _hip._COPY_MIN for x in xs]
-    if large.count(True) < 2:
-        return [fam.f64(x) for x in xs]
-    place, out = _hip.FIRST, []
-    for x, staged in zip(xs, large):
-        out.append(fam.f64(x, place))
-        if staged:
-            place = _hip.FOLLOWING
-        elif is_torch(x):  # may have queued a conversion
-            place = _hip.FIRST
     return out
 
 
@@ -185,7 +167,7 @@ class _TorchFamily:
     def stream(self):
         return torch.cuda.current_stream().cuda_stream
 
-    def f64(self, x, place=_hip.ALONE):
+    def f64(self, x):
         """float64 device tensor with contiguous rows holding x's values;
         never aliases a NumPy input."""
         if is_torch(x):
@@ -196,12 +178,15 @@ class _TorchFamily:
                 t = t.to(self.dev)
         else:
             a = np.ascontiguousarray(np.asarray(x, dtype=np.float64))
-            t = _numpy_to_torch(a, self.dev, place)
+            t = _numpy_to_torch(a, self.dev)
         if t.dim() >= 1 and t.numel() > 0 and t.stride(-1) != 1:
             t = t.contiguous()
         if t.dim() == 2 and t.numel() > 0 and t.stride(0) < max(t.shape[1], 1):
             t = t.contiguous()
         return t
+
+    def f64s(self, *xs):
+        return [self.f64(x) for x in xs]
 
     def empty(self, shape, dtype=np.float64):
         return torch.empty(shape, dtype=_TORCH_DTYPES[np.dtype(dtype)], device=self.dev)
@@ -289,6 +274,21 @@ class _HipFamily:
         if is_torch(x):  # matmul_numpy takes any array-like
             x = x.detach().cpu().numpy()
         return _hip.DeviceArray.from_numpy(np.asarray(x, dtype=np.float64), place)
+
+    def f64s(self, *xs):
+        """f64 of each: a staged upload behind another one does not wait for
+        it, so that its host copy overlaps the other's transfer."""
+        large = [isinstance(x, np.ndarray) and 8 * x.size >= _hip._COPY_MIN for x in xs]
+        if large.count(True) < 2:
+            return [self.f64(x) for x in xs]
+        place, out = _hip.FIRST, []
+        for x, staged in zip(xs, large):
+            out.append(self.f64(x, place))
+            if staged:
+                place = _hip.FOLLOWING
+            elif is_torch(x):  # may have queued a conversion
+                place = _hip.FIRST
+        return out
 
     def empty(self, shape, dtype=np.float64):
         return _hip.DeviceArray(shape, dtype)

@@ -197,7 +197,7 @@ def _matmul_ondevice_numpy(fam, A, B, safe_mode, accumulation, n_hi, n_lo):
     _check_safe_mode(safe_mode)
 
     def whole():
-        return _matmul_ondevice(fam, *D.f64s(fam, A, B), safe_mode, accumulation,
+        return _matmul_ondevice(fam, *fam.f64s(A, B), safe_mode, accumulation,
                                 n_hi, n_lo).numpy()
 
     if _kbound_reasons(K, 24 - rho_f32(K), "large for FP32 extraction"):
@@ -205,7 +205,7 @@ def _matmul_ondevice_numpy(fam, A, B, safe_mode, accumulation, n_hi, n_lo):
     order = _lib.ORDER_BLOCK64 if accumulation == "host" else _lib.ORDER_2SUM
     lib, rt, st = _lib.load(), _hip._rt(), _hip.compute_stream()
     h = (N // 2 + 63) // 64 * 64
-    Bt, At = D.f64s(fam, B, A[:h])
+    Bt, At = fam.f64s(B, A[:h])
     held, done = [Bt], []
     out = np.empty((N, M))
     fl = 0
@@ -301,13 +301,13 @@ def matmul(A, B, n_slices=8, safe_mode="raise", pipeline="host",
         n_hi, n_lo = _resolve_precision(precision)
         if not want_torch and _numpy_halves_ok(A, B):
             return _matmul_ondevice_numpy(fam, A, B, safe_mode, accumulation, n_hi, n_lo)
-        At, Bt = D.f64s(fam, A, B)
+        At, Bt = fam.f64s(A, B)
         C = _matmul_ondevice(fam, At, Bt, safe_mode, accumulation, n_hi, n_lo)
         return fam.out(C, want_torch)
     if pipeline != "host":
         raise ValueError(
             f"Unknown pipeline={pipeline!r}; expected 'host' or 'ondevice'.")
-    At, Bt = D.f64s(fam, A, B)
+    At, Bt = fam.f64s(A, B)
     C = _matmul_host(fam, At, Bt, n_slices, safe_mode, _lib.ORDER_HOST_JAX)
     return fam.out(C, False)
 
@@ -323,7 +323,7 @@ def matmul_numpy(A_f64, B_f64, n_slices=8, safe_mode="raise", pipeline="host",
     if pipeline == "ondevice" and not want_torch and _numpy_halves_ok(A_f64, B_f64):
         n_hi, n_lo = _resolve_precision(precision)
         return _matmul_ondevice_numpy(fam, A_f64, B_f64, safe_mode, "host", n_hi, n_lo)
-    At, Bt = D.f64s(fam, A_f64, B_f64)
+    At, Bt = fam.f64s(A_f64, B_f64)
     if pipeline == "ondevice":
         n_hi, n_lo = _resolve_precision(precision)
         C = _matmul_ondevice(fam, At, Bt, safe_mode, "host", n_hi, n_lo)

@@ -129,7 +129,7 @@ def fused_ozaki_matmul(A_f64, B_f64, rho, n_hi, n_lo, *, bm=128, bk=128, bn=128)
     from . import lowlevel as ll
     want_torch = D.is_torch(A_f64)
     fam = D.family(True)  # the stage-level planes are torch tensors
-    A, B = D.f64s(fam, A_f64, B_f64)
+    A, B = fam.f64s(A_f64, B_f64)
     if A.shape[1] != B.shape[0]:
         raise ValueError(f"incompatible shapes {tuple(A.shape)} and {tuple(B.shape)}")
     pa = ll.extract(A, 0, int(rho), n_hi, n_lo)

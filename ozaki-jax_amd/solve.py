@@ -123,7 +123,7 @@ def residual(A, x, b, precision="high", accumulation="bf16_interleaved",
     want_torch = D.is_torch(A)
     _validate_residual_inputs(A, x, b)
     fam = D.family(want_torch)
-    At, xt, bt = D.f64s(fam, A, x, b)
+    At, xt, bt = fam.f64s(A, x, b)
     vec = xt.dim() == 1
     if vec:
         xt = fam.column(xt)
@@ -198,7 +198,7 @@ def _solve_numpy(A, b, precision, max_iterations, residual_mode):
     b = np.asarray(b, dtype=np.float64)
     vec = b.ndim == 1
     n = A.shape[0]
-    At, bt = D.f64s(fam, A, b[:, None] if vec else b)
+    At, bt = fam.f64s(A, b[:, None] if vec else b)
     nc = bt.shape[1]
     if n == 0 or nc == 0:
         return np.zeros(b.shape)

@@ -135,13 +135,12 @@ def test_copies_do_not_wait_for_another_threads_stream(ozk, way, mib):
     assert early, "the copy waited for the other thread's stream"
 
 
-@pytest.mark.parametrize("torch_family", [False, True])
-def test_f64s_by_place(ozk, monkeypatch, torch_family):
+def test_f64s_by_place(ozk, monkeypatch):
     """Which uploads are staged, and which of them follow another without a
     wait: sizes around the thresholds, alone and in rows."""
     import torch
     from ozaki_jax_amd import _device as D, _hip
-    fam = D.family(torch_family)
+    fam = D.family(False)
     seen = []
     to_device = _hip._Stager.to_device
 
@@ -157,14 +156,12 @@ def test_f64s_by_place(ozk, monkeypatch, torch_family):
     rows = [([one], []), ([big], [False]), ([four, small], []),
             ([one, four], [False, True]), ([one, small, four], [False, True]),
             ([four.astype(np.float32), one, big], [False, True, True])]
-    if torch_family:
-        rows.append(([one, tensor, four, one], [False, False, True]))
+    rows.append(([one, tensor, four, one], [False, True, False, True]))
     for xs, want in rows:
         del seen[:]
         case(f"f64s of {[x.nbytes if isinstance(x, np.ndarray) else 'tensor' for x in xs]}")
-        out = D.f64s(fam, *xs)
+        out = fam.f64s(*xs)
         assert [f for _, f in seen] == want
         for x, t in zip(xs, out):
-            got = t.cpu().numpy() if torch_family else t.numpy()
             x = x if isinstance(x, np.ndarray) else x.cpu().numpy()
-            assert np.array_equal(got, x.astype(np.float64))
+            assert np.array_equal(t.numpy(), x.astype(np.float64))
