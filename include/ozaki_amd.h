@@ -319,8 +319,9 @@ int ozk_matmul_early_flags(const double* A, int64_t lda, const double* B,
  * OZK_FLAGS_READY when the extraction has run and the GEMM starts.  Against
  * ozk_matmul_early_flags this saves a clearing kernel, a copy and an event.
  * Both words belong to one call at a time; after OZK_ERR_HIP neither may be
- * used again (other errors come before anything is queued).  ozk_wait_flag_word waits for a published word and returns its flags;
- * it ends with OZK_ERR_HIP on a stream that failed, is being captured or drained
+ * used again (other errors come before anything is queued).
+ * ozk_wait_flag_word waits for a published word and returns its flags; it
+ * ends with OZK_ERR_HIP on a stream that failed, is being captured or drained
  * without publishing. */
 int ozk_matmul_flag_word(const double* A, int64_t lda, const double* B,
                          int64_t ldb, double* C, int64_t ldc, int64_t N,

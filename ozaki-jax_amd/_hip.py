@@ -141,8 +141,9 @@ class _Runtime:
 # (_Stager); smaller ones are as fast as the runtime's own copies.  So is an
 # upload below _ALONE_MIN that no other follows or precedes, since staging gains
 # from the overlap of two (host products of an array of 1, 2, 4, 8, 12 MiB with a
-# small one: 177, 211, 321, 535, 715 us; staged 190, 240, 346, 490, 610).  Those above _SLOTS * _SLOT bytes take the larger slots.  Products whose
-# halves reach _STAGE_MIN bytes run in two halves (matmul).
+# small one: 177, 211, 321, 535, 715 us; staged 190, 240, 346, 490, 610).  Those
+# above _SLOTS * _SLOT bytes take the larger slots.  Products whose halves reach
+# _STAGE_MIN bytes run in two halves (matmul).
 _COPY_MIN = 1 << 20
 _ALONE_MIN = 6 << 20
 ALONE, FIRST, FOLLOWING = 0, 1, 2  # place of an upload among several (from_numpy)
@@ -476,9 +477,9 @@ def _release_at_exit():
     work end, then release what this package holds in the runtime (the
     staging buffers and their events, the rocBLAS handle, the compute stream,
     the pool's cached blocks, and through _exit_hooks what other modules keep),
-    so that none of it is left for the runtime's static destructors.  The runtime and the pool stay: blocks that arrays
-    release later are freed at once.  Errors are ignored: the runtime may be
-    unusable by then."""
+    so that none of it is left for the runtime's static destructors.  The
+    runtime and the pool stay: blocks that arrays release later are freed at
+    once.  Errors are ignored: the runtime may be unusable by then."""
     with _state_lock:
         st = dict(_state)
         for k in st:

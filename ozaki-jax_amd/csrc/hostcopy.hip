@@ -16,10 +16,10 @@
 // stream has drained: queued behind kernels they would keep the slots, and the
 // DMA engine they are queued on, from everyone.  (The second of two uploads in a
 // row goes behind the first all the same: a product of 400^3 NumPy arrays takes
-// 230 to 255 us, 265 where it waits, 225 where neither does.)  The small copy down, a kernel, does not
-// wait either, which would cost it about 40 us (56 -> 95 at 1 MiB, 235 -> 330 at
-// 8): it holds the memory from its launch on, and a caller that finds it held
-// takes the runtime's own copy.
+// 230 to 255 us, 265 where it waits, 225 where neither does.)  The small copy
+// down, a kernel, does not wait either, which would cost it about 40 us (56 -> 95
+// at 1 MiB, 235 -> 330 at 8): it holds the memory from its launch on, and a
+// caller that finds it held takes the runtime's own copy.
 #include <atomic>
 #include <condition_variable>
 #include <mutex>

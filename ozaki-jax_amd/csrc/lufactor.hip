@@ -66,12 +66,13 @@ __device__ __forceinline__ uint32_t lu_wave_reduce(uint32_t u) {
 // the rank-1 update: 0.9 us at one row slot, 28.8 a panel.  What taller panels
 // take beyond that (34.9 us at 2 slots, 42.4 at 4, 51.9 at 6, 76.2 at 8) is the
 // vector work and the loads of one CU, and at 7 and 8 slots, and from 5 on
-// without 16-byte rows, registers spilled to scratch.  The steps run as a rolled loop: unrolled over the 32
-// columns the kernel was 28000 instructions, and fetching that much
-// straight-line code (200 KB, over the 64 KB instruction cache) cost about
-// a sixth of every short step and more of the tall ones.  The loop needs the active column
-// in a fixed register, so each step rotates a row's registers by one: the
-// updated columns move down and the finished L entry enters at the end.
+// without 16-byte rows, registers spilled to scratch.  The steps run as a rolled
+// loop: unrolled over the 32 columns the kernel was 28000 instructions, and
+// fetching that much straight-line code (200 KB, over the 64 KB instruction
+// cache) cost about a sixth of every short step and more of the tall ones.  The
+// loop needs the active column in a fixed register, so each step rotates a row's
+// registers by one: the updated columns move down and the finished L entry
+// enters at the end.
 // Measured with the row slots a compile-time count, the loads and stores
 // four lanes a row and the permutation composed in parallel (us a panel,
 // unrolled -> rolled): 4096 rows 108 -> 83, 2048 71 -> 45, 512 46 -> 30; n =
